@@ -1,0 +1,159 @@
+"""Bulk calls that sort their batch by table region first (partition.hpp):
+sizes around the passes' edges (one and two sorting passes, ragged tiles, a
+last region of few windows), duplicate-heavy and skewed batches (segments
+that overflow), invalid keys, limited probing, batches on top of stored keys,
+and tables that more than one stream modifies."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from datagen import dev_empty, dtype, from_dev, to_dev, tomb, uniform_values, unique_keys
+
+pytestmark = pytest.mark.gpu
+
+S_NONE, S_PLE, S_INVALID_KEY, S_DUP, S_NOT_FOUND = 0, 2, 8, 16, 32
+SENTINEL = 0x5A5A5A5A
+
+
+def _batch(n, bits, shape, seed):
+    """n keys: distinct, or with the duplicates `shape` names."""
+    rng = np.random.default_rng(seed)
+    keys = unique_keys(n, bits, seed)
+    if shape == "repeats":          # every eighth key twice
+        keys[: n // 8] = keys[n - n // 8:]
+        rng.shuffle(keys)
+    elif shape == "hot":            # two keys take half of the batch
+        keys[::3] = keys[1]
+        keys[1::7] = keys[2]
+    elif shape == "few":            # about fifty copies of each key: region segments overflow
+        keys = keys[rng.integers(0, max(1, n // 50), n)]
+    elif shape == "invalid":
+        keys[::997] = 0
+        keys[3::1009] = tomb(bits)
+    return np.ascontiguousarray(keys)
+
+
+def _value_of(keys, bits):
+    x = keys.astype(np.uint64) * np.uint64(0x9E3779B97F4A7C15) + np.uint64(0x7F4A7C15)
+    return (x >> np.uint64(64 - bits)).astype(dtype(bits)) if bits == 32 else x
+
+
+def _valid(keys, bits):
+    return (keys != 0) & (keys != tomb(bits))
+
+
+def _status_counts(keys, st, bits):
+    """Per distinct valid key: how many `none` among its statuses."""
+    ok = _valid(keys, bits)
+    uniq, inv = np.unique(keys[ok], return_inverse=True)
+    return np.bincount(inv, weights=(st[ok] == S_NONE), minlength=len(uniq))
+
+
+@pytest.mark.parametrize("kb,vb,cg,n,load,shape", [
+    (64, 64, 8, 1 << 20, 0.9, "distinct"),
+    (64, 64, 8, (1 << 21) + 4095, 0.93, "repeats"),
+    (64, 64, 8, 5_000_001, 0.9, "distinct"),      # more than 1024 regions: two passes
+    (64, 64, 8, 5_000_001, 0.9, "hot"),
+    (64, 64, 8, 4_500_000, 0.9, "few"),
+    (64, 64, 16, 2_000_003, 0.8, "invalid"), (64, 64, 4, 1_500_001, 0.9, "repeats"),
+    (32, 32, 16, 12_000_001, 0.9, "distinct"), (32, 32, 16, (1 << 21) - 1, 0.95, "few"),
+    (32, 32, 8, 1 << 20, 0.8, "hot"), (32, 32, 8, 9_000_007, 0.9, "repeats"), (32, 32, 4, 1 << 20, 0.9, "invalid"),
+    (32, 64, 8, 1_234_567, 0.9, "repeats"), (64, 32, 8, 6_400_000, 0.9, "hot"),
+])
+@pytest.mark.parametrize("statuses", [False, True])
+def test_insert(cuda, kb, vb, cg, n, load, shape, statuses):
+    from warpcore_amd.tables import SingleValueHashTable
+    keys = _batch(n, kb, shape, seed=n + cg)
+    vals = _value_of(keys, vb)
+    t = SingleValueHashTable(math.ceil(n / load), kb, vb, cg_size=cg)
+    st = dev_empty(n, 32, 0x77)
+    t.insert(to_dev(keys), to_dev(vals), status_out=st if statuses else None)
+    valid = _valid(keys, kb)
+    uniq = np.unique(keys[valid])
+    assert t.size() == len(uniq)
+    word = (S_DUP if len(uniq) < valid.sum() else 0) | (S_INVALID_KEY if not valid.all() else 0)
+    assert int(t.pop_status()) == word
+    if statuses:
+        got = from_dev(st, np.uint32)
+        assert (got[~valid] == S_INVALID_KEY).all()
+        assert set(np.unique(got[valid])) <= {S_NONE, S_DUP}
+        assert (_status_counts(keys, got, kb) == 1).all()
+    out, found = dev_empty(n, vb, SENTINEL), dev_empty(n, 32, 0x77)
+    t.retrieve(to_dev(keys), out, status_out=found)
+    found = from_dev(found, np.uint32)
+    assert (found[valid] == S_NONE).all() and (found[~valid] == S_INVALID_KEY).all()
+    np.testing.assert_array_equal(from_dev(out, dtype(vb))[valid], vals[valid])
+    absent = unique_keys(100_000, kb, seed=3, exclude=uniq)
+    out = dev_empty(len(absent), vb, SENTINEL)
+    t.retrieve(to_dev(absent), out, status_out=st[: len(absent)])
+    assert (from_dev(st[: len(absent)], np.uint32) == S_NOT_FOUND).all()
+    assert (from_dev(out, dtype(vb)) == SENTINEL).all()
+
+
+@pytest.mark.parametrize("kb,cg", [(64, 8), (32, 16)])
+def test_insert_limited_probing(cuda, kb, cg):
+    """One window per key: keys past a full first window report
+    probing_length_exceeded, and exactly the others are stored."""
+    from warpcore_amd.tables import SingleValueHashTable
+    n = 3_000_017
+    keys = unique_keys(n, kb, seed=5)
+    t = SingleValueHashTable(math.ceil(n / 0.95), kb, kb, cg_size=cg)
+    st = dev_empty(n, 32, 0x77)
+    t.insert(to_dev(keys), to_dev(keys), status_out=st, probing_length=cg)
+    st = from_dev(st, np.uint32)
+    assert set(np.unique(st)) == {S_NONE, S_PLE}
+    assert int(t.pop_status()) == S_PLE
+    assert t.size() == (st == S_NONE).sum()
+    out, found = dev_empty(n, kb, SENTINEL), dev_empty(n, 32, 0x77)
+    t.retrieve(to_dev(keys), out, status_out=found, probing_length=cg)
+    found = from_dev(found, np.uint32)
+    np.testing.assert_array_equal(found == S_NONE, st == S_NONE)
+
+
+@pytest.mark.parametrize("kb,vb,cg", [(64, 64, 8), (32, 32, 8)])
+def test_insert_on_stored_keys(cuda, kb, vb, cg):
+    """Half of the keys stored one small batch at a time before (another
+    kernel, other slot orders), some erased; then all of them at once."""
+    from warpcore_amd.tables import SingleValueHashTable
+    n = 1_300_003
+    keys = unique_keys(n, kb, seed=9)
+    old = uniform_values(n, vb, seed=10)
+    t = SingleValueHashTable(math.ceil(n / 0.8), kb, vb, cg_size=cg)
+    half = n // 2
+    for lo in range(0, half, 100_000):
+        hi = min(lo + 100_000, half)
+        t.insert(to_dev(keys[lo:hi]), to_dev(old[lo:hi]))
+    t.erase(to_dev(keys[:1000]))
+    st = dev_empty(n, 32, 0x77)
+    t.insert(to_dev(keys), to_dev(_value_of(keys, vb)), status_out=st)
+    st = from_dev(st, np.uint32)
+    assert (st[:1000] == S_NONE).all() and (st[1000:half] == S_DUP).all() and (st[half:] == S_NONE).all()
+    assert t.size() == n
+    out = dev_empty(n, vb, SENTINEL)
+    t.retrieve(to_dev(keys), out)
+    np.testing.assert_array_equal(from_dev(out, dtype(vb)), _value_of(keys, vb))
+
+
+def test_inserts_from_two_streams(cuda):
+    """Batches inserted on two streams without synchronization: every key is
+    stored, whichever batch was partitioned."""
+    from warpcore_amd.tables import SingleValueHashTable
+    n = 2_000_000
+    keys = unique_keys(3 * n, 64, seed=21)
+    vals = _value_of(keys, 64)
+    kd, vd = to_dev(keys), to_dev(vals)
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    t = SingleValueHashTable(math.ceil(3 * n / 0.85), 64, 64)
+    torch.cuda.synchronize()
+    for round_ in range(3):   # the first round's insert on `a` is partitioned, the one on `b` waits for it
+        t.init(stream=a)
+        for i, s in enumerate((a, b, a)):
+            t.insert(kd[i * n:(i + 1) * n], vd[i * n:(i + 1) * n], stream=s)
+        torch.cuda.synchronize()
+        assert t.size() == 3 * n
+        out = torch.zeros_like(vd)
+        t.retrieve(kd, out, stream=a)
+        torch.cuda.synchronize()
+        assert torch.equal(out, vd)

@@ -1,0 +1,148 @@
+// Who may modify a table while a bulk insert rewrites it.
+//
+// The partitioned inserts (partition.hpp) write whole regions of a table
+// back with plain stores, so nothing else may modify the table meanwhile;
+// every other path claims slots by compare-and-swap and runs beside anything.
+// MutationTracker decides which of the two a bulk call takes:
+//
+// - Every bulk call that modifies the table notes its stream. A call may run
+//   exclusively while all of them used that one stream, which then orders
+//   them. A second stream, a call under capture (its graph may be replayed at
+//   any time), the per-thread default stream (one handle, many streams), and
+//   a copy or a view of the table handed out (user kernels may modify the
+//   table through the device calls) end that; the calls that follow use the
+//   compare-and-swap paths.
+// - An exclusive call leaves an event behind its kernels. A later modifying
+//   call on another stream waits for it on the device, and handing out a copy
+//   or a view, or noting a call under capture, waits for it on the host.
+// - init() starts over (it fills the whole table, so a modification still
+//   running on another stream would be a race with it already), except for
+//   copies, views and graphs, which stay.
+#pragma once
+
+#include "base.hpp"
+
+#include <mutex>
+#include <new>
+
+namespace warpcore {
+namespace detail {
+
+class MutationTracker {
+    struct State {
+        std::mutex mu;
+        bool any = false;      // `stream` is the one that ordered every modification so far
+        bool mixed = false;    // more than one stream since the last init()
+        bool shared = false;   // a copy, a view or a graph may modify the table
+        hipStream_t stream = nullptr;
+        hipEvent_t fence = nullptr;   // behind the last exclusive call
+        bool fenced = false;
+        hipStream_t fence_stream = nullptr;
+    };
+
+public:
+    WC_H MutationTracker() noexcept : s_(new (std::nothrow) State) {}
+    // a shallow copy of the table: it shares the state, which its owner destroys
+    WC_HD MutationTracker(const MutationTracker& o) noexcept : s_(o.s_) { share(); }
+    WC_H MutationTracker(MutationTracker&& o) noexcept : s_(o.s_) {}
+    MutationTracker& operator=(const MutationTracker&) = delete;
+
+    WC_H void destroy() noexcept {   // by the table that owns the state
+        if (s_ == nullptr) return;
+        if (s_->fence != nullptr) (void)hipEventDestroy(s_->fence);
+        delete s_;
+        s_ = nullptr;
+    }
+
+    WC_HD void share() const noexcept {
+#if !defined(__HIP_DEVICE_COMPILE__)
+        if (s_ == nullptr) return;
+        std::lock_guard<std::mutex> lock(s_->mu);
+        share_locked();
+#endif
+    }
+    WC_H void restart() const noexcept {
+        if (s_ == nullptr) return;
+        std::lock_guard<std::mutex> lock(s_->mu);
+        s_->any = false;
+        s_->mixed = false;
+    }
+    // a modification on `stream` that runs beside others
+    WC_H void note(hipStream_t stream) const noexcept {
+        if (s_ == nullptr) return;
+        std::lock_guard<std::mutex> lock(s_->mu);
+        (void)note_locked(stream);
+    }
+
+    // One exclusive call: granted() says whether the kernels enqueued while
+    // this object lives may assume that nothing else modifies the table.
+    // Modifying calls of other host threads wait until it is gone.
+    class Exclusive {
+    public:
+        WC_H Exclusive(const MutationTracker& t, hipStream_t stream) noexcept : s_(t.s_), stream_(stream) {
+            if (s_ == nullptr) return;
+            s_->mu.lock();
+            granted_ = t.note_locked(stream);
+            if (granted_ && s_->fence == nullptr &&
+                hipEventCreateWithFlags(&s_->fence, hipEventDisableTiming) != hipSuccess) {
+                (void)hipGetLastError();
+                s_->fence = nullptr;
+                granted_ = false;
+            }
+        }
+        Exclusive(const Exclusive&) = delete;
+        Exclusive& operator=(const Exclusive&) = delete;
+        WC_H ~Exclusive() noexcept {
+            if (s_ == nullptr) return;
+            if (used_) {
+                if (hipEventRecord(s_->fence, stream_) == hipSuccess) {
+                    s_->fenced = true;
+                    s_->fence_stream = stream_;
+                } else {   // no event to wait for: the kernels end here
+                    (void)hipGetLastError();
+                    (void)hipStreamSynchronize(stream_);
+                }
+            }
+            s_->mu.unlock();
+        }
+        bool granted() const noexcept { return granted_; }
+        void use() noexcept { used_ = true; }   // exclusive kernels were enqueued
+
+    private:
+        State* s_;
+        hipStream_t stream_;
+        bool granted_ = false, used_ = false;
+    };
+
+private:
+    WC_H void share_locked() const noexcept {
+        s_->shared = true;
+        if (!s_->fenced) return;
+        // also called while some stream of this thread is captured, where a
+        // host wait needs the relaxed mode
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        const bool exchanged = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+        (void)hipEventSynchronize(s_->fence);
+        if (exchanged) (void)hipThreadExchangeStreamCaptureMode(&mode);
+        s_->fenced = false;
+    }
+    // whether `stream` orders every modification
+    WC_H bool note_locked(hipStream_t stream) const noexcept {
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) {
+            (void)hipGetLastError();
+            share_locked();
+            return false;
+        }
+        if (s_->fenced && s_->fence_stream != stream) (void)hipStreamWaitEvent(stream, s_->fence, 0);
+        if (stream == hipStreamPerThread || (s_->any && s_->stream != stream)) s_->mixed = true;
+        s_->any = true;
+        s_->stream = stream;
+        return !s_->mixed && !s_->shared;
+    }
+
+    State* s_;
+};
+
+}  // namespace detail
+}  // namespace warpcore

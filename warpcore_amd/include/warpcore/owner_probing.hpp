@@ -91,15 +91,30 @@ WC_D void owner_load_pair(const T* p, T (&out)[SPL]) noexcept {
     }
 }
 
-// Inserts of keys_in[first .. end) by the calling wavefront (all 64 lanes
+// Keys and values of an insert as plain arrays; position(i) is where key i's
+// status goes.
+template<class K, class V, bool HasValues>
+struct ArrayInput {
+    const K* __restrict__ keys;
+    const V* __restrict__ values;
+    WC_D K key(index_t i) const noexcept { return keys[i]; }
+    WC_D V value(index_t i) const noexcept {
+        if constexpr (HasValues) return values[i];
+        else return V{};
+    }
+    WC_D static index_t position(index_t i) noexcept { return i; }
+};
+
+// Inserts of keys first .. end of `in` by the calling wavefront (all 64 lanes
 // call this with the same range). `lds` holds 64 entries of this wave.
-// Single-value cores only (insert_refill_range covers multi-value cores).
-template<class Core, class StatusHandler, class W, bool HasValues, unsigned SPL = 1>
-WC_D void insert_owner_range(const typename Core::key_type* __restrict__ keys_in,
-                             const typename Core::value_type* __restrict__ values_in, index_t first, index_t end,
-                             const Core& core, index_t budget,
-                             typename StatusHandler::base_type* __restrict__ status_out,
-                             OwnerEntry<typename Core::key_type, W>* lds, DeferredJoin& join) {
+// SkipFirst: every key's first window is known to be full, not to hold the
+// key, and marked in the overflow filter; its walk starts at the second
+// window (single-value cores: a multi-value core counts the key's values in
+// every window).
+template<class Core, class StatusHandler, class W, bool HasValues, unsigned SPL, bool SkipFirst, class Input>
+WC_D void insert_owner_from(const Input& in, index_t first, index_t end, const Core& core, index_t budget,
+                            typename StatusHandler::base_type* __restrict__ status_out,
+                            OwnerEntry<typename Core::key_type, W>* lds, DeferredJoin& join) {
     using K = typename Core::key_type;
     using V = typename Core::value_type;
     using Probe = typename Core::insert_probe_type;
@@ -110,6 +125,7 @@ WC_D void insert_owner_range(const typename Core::key_type* __restrict__ keys_in
     constexpr unsigned CG = WIN / SPL;                     // lanes per group
     static_assert(CG >= 2 && CG <= 64 && (CG & (CG - 1)) == 0, "groups of 2..64 lanes");
     constexpr bool multi = is_multi_value_core<Core>::value;
+    static_assert(!(multi && SkipFirst), "multi-value walks start at the first window");
     static_assert(SPL == 1 || (SPL == 2 && !multi && sizeof(Probe) == 8 && !std::is_same<Probe, K>::value),
                   "two slots per lane: packed 8-byte slots of single-value cores");
     constexpr bool keep_seen = !std::is_same<Probe, K>::value;
@@ -125,7 +141,7 @@ WC_D void insert_owner_range(const typename Core::key_type* __restrict__ keys_in
     if (end <= first) return;
     if (!core.ready()) {
         for (index_t i = first + lane; i < end; i += 64)
-            StatusHandler::handle(Status::not_initialized(), status_out, i);
+            StatusHandler::handle(Status::not_initialized(), status_out, in.position(i));
         return;
     }
 
@@ -146,8 +162,8 @@ WC_D void insert_owner_range(const typename Core::key_type* __restrict__ keys_in
     index_t npos = cursor + lane;
     bool nhas = npos < end;
     if (nhas) {
-        nk = keys_in[npos];
-        if constexpr (HasValues) nv = values_in[npos];
+        nk = in.key(npos);
+        if constexpr (HasValues) nv = in.value(npos);
     }
     cursor += 64;
 
@@ -158,7 +174,7 @@ WC_D void insert_owner_range(const typename Core::key_type* __restrict__ keys_in
             if constexpr (multi)
                 if (count > 0) st = st + Status::duplicate_key();
             join(st);
-            StatusHandler::handle(st, status_out, pos);
+            StatusHandler::handle(st, status_out, in.position(pos));
             phase = kFree;
         } else {
             const W nw = w + step;
@@ -183,9 +199,20 @@ WC_D void insert_owner_range(const typename Core::key_type* __restrict__ keys_in
                 rnd = 0;
                 count = 0;
                 phase = kLoad;
+                if constexpr (SkipFirst) {
+                    if (budget <= 1) {
+                        join(Status::probing_length_exceeded());
+                        StatusHandler::handle(Status::probing_length_exceeded(), status_out, in.position(pos));
+                        phase = kFree;
+                    } else {
+                        const W nw = w + step;
+                        w = nw >= p ? W(nw - p) : nw;
+                        rnd = 1;
+                    }
+                }
             } else {
                 join(Status::invalid_key());
-                StatusHandler::handle(Status::invalid_key(), status_out, pos);
+                StatusHandler::handle(Status::invalid_key(), status_out, in.position(pos));
             }
         }
         const std::uint64_t taken = ballot(take);
@@ -194,8 +221,8 @@ WC_D void insert_owner_range(const typename Core::key_type* __restrict__ keys_in
                 npos = cursor + lanes_below(taken);
                 nhas = npos < end;
                 if (nhas) {
-                    nk = keys_in[npos];
-                    if constexpr (HasValues) nv = values_in[npos];
+                    nk = in.key(npos);
+                    if constexpr (HasValues) nv = in.value(npos);
                 }
             }
             cursor += index_t(__builtin_popcountll(taken));
@@ -239,14 +266,14 @@ WC_D void insert_owner_range(const typename Core::key_type* __restrict__ keys_in
                     Status fin = st;
                     core.finish_insert(index_t(w) * WIN + lead, val, Core::publishes_value, fin, join);
                     if (count == 0) ++new_keys;
-                    StatusHandler::handle(st, status_out, pos);
+                    StatusHandler::handle(st, status_out, in.position(pos));
                     phase = kFree;
                 } else if (code == 0 || code == 2) {
                     if (code == 2) count += 1;
                     if (count >= index_t(core.max_values)) {
                         const Status full = Status::duplicate_key() + Status::max_values_for_key_reached();
                         join(full);
-                        StatusHandler::handle(full, status_out, pos);
+                        StatusHandler::handle(full, status_out, in.position(pos));
                         phase = kFree;
                     } else {
                         emp &= Bits(emp - 1);
@@ -262,7 +289,7 @@ WC_D void insert_owner_range(const typename Core::key_type* __restrict__ keys_in
                     core.finish_insert(index_t(w) * WIN + lead, val, code == 1 && Core::publishes_value, st, join);
                     record_slot(core, index_t(w) * WIN + lead, pos, code == 1);
                     if (code == 2) join(Status::duplicate_key());
-                    StatusHandler::handle(st, status_out, pos);
+                    StatusHandler::handle(st, status_out, in.position(pos));
                     phase = kFree;
                 } else if (code == 0) {   // another key took the slot: the window's next EMPTY slot
                     emp &= Bits(emp - 1);
@@ -296,7 +323,7 @@ WC_D void insert_owner_range(const typename Core::key_type* __restrict__ keys_in
                 if (count >= index_t(core.max_values)) {
                     const Status full = Status::duplicate_key() + Status::max_values_for_key_reached();
                     join(full);
-                    StatusHandler::handle(full, status_out, pos);
+                    StatusHandler::handle(full, status_out, in.position(pos));
                     phase = kFree;
                 } else if (empty != 0) {
                     emp = empty;
@@ -314,7 +341,7 @@ WC_D void insert_owner_range(const typename Core::key_type* __restrict__ keys_in
                     core.finish_insert(at, val, false, st, join);
                     record_slot(core, at, pos, false);
                     join(Status::duplicate_key());
-                    StatusHandler::handle(st, status_out, pos);
+                    StatusHandler::handle(st, status_out, in.position(pos));
                     phase = kFree;
                 } else if (empty != 0) {
                     emp = empty;
@@ -327,6 +354,17 @@ WC_D void insert_owner_range(const typename Core::key_type* __restrict__ keys_in
         }
     }
     if constexpr (multi) core.add_keys(new_keys);
+}
+
+template<class Core, class StatusHandler, class W, bool HasValues, unsigned SPL = 1>
+WC_D void insert_owner_range(const typename Core::key_type* __restrict__ keys_in,
+                             const typename Core::value_type* __restrict__ values_in, index_t first, index_t end,
+                             const Core& core, index_t budget,
+                             typename StatusHandler::base_type* __restrict__ status_out,
+                             OwnerEntry<typename Core::key_type, W>* lds, DeferredJoin& join) {
+    const ArrayInput<typename Core::key_type, typename Core::value_type, HasValues> in{keys_in, values_in};
+    insert_owner_from<Core, StatusHandler, W, HasValues, SPL, false>(in, first, end, core, budget, status_out, lds,
+                                                                     join);
 }
 
 // Lookups of keys_in[first .. end) by the calling wavefront. A hit is

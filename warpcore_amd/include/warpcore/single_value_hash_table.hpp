@@ -22,6 +22,8 @@
 #include "lockstep_probing.hpp"
 #include "refill_probing.hpp"
 #include "engine.hpp"
+#include "mutation.hpp"
+#include "partition.hpp"
 #include "probing_schemes.hpp"
 #include "status.hpp"
 #include "storage.hpp"
@@ -51,6 +53,7 @@ struct SingleValueView {
     using probe_slot_type = Slot;
     static constexpr bool packed = is_packed_pair<Slot>();
     static constexpr bool publishes_value = packed;
+    static constexpr RegionOp region_op = RegionOp::assign;   // partitioned inserts (partition.hpp)
 
     Slot* slots;
     Status* status;
@@ -469,18 +472,19 @@ public:
             if (table_.capacity() != 0 && hipMalloc(&filter_, filter_bytes()) != hipSuccess) filter_ = nullptr;
         }
         assign_status(table_.status() + temp_.status());
+        detail::WorkspacePool::instance().add_user();
         if (!no_init) init();
     }
 
     WC_HD SingleValueHashTable(const SingleValueHashTable& o) noexcept
         : status_(o.status_), table_(o.table_), temp_(o.temp_), seed_(o.seed_),
           is_initialized_(o.is_initialized_), is_copy_(true), geo_(o.geo_), filter_(o.filter_),
-          filter_valid_(o.filter_valid_) {}
+          filter_valid_(o.filter_valid_), mutations_(o.mutations_) {}
 
     WC_H SingleValueHashTable(SingleValueHashTable&& o) noexcept
         : status_(o.status_), table_(std::move(o.table_)), temp_(std::move(o.temp_)), seed_(o.seed_),
           is_initialized_(o.is_initialized_), is_copy_(o.is_copy_), geo_(o.geo_), filter_(o.filter_),
-          filter_valid_(o.filter_valid_) {
+          filter_valid_(o.filter_valid_), mutations_(std::move(o.mutations_)) {
         o.is_copy_ = true;
     }
 
@@ -488,6 +492,10 @@ public:
 #if !defined(__HIP_DEVICE_COMPILE__)
         if (!is_copy_ && status_ != nullptr) (void)hipFree(status_);
         if (!is_copy_ && filter_ != nullptr) (void)hipFree(filter_);
+        if (!is_copy_) {
+            mutations_.destroy();
+            detail::WorkspacePool::instance().remove_user();
+        }
 #endif
     }
 
@@ -495,6 +503,7 @@ public:
     WC_H void init(key_type seed, hipStream_t stream = 0) noexcept {
         is_initialized_ = false;
         seed_ = seed;
+        mutations_.restart();
         if (!table_.status().has_not_initialized() && !temp_.status().has_not_initialized()) {
             table_.init_keys(empty_key(), stream);
             if (filter_ != nullptr)
@@ -512,17 +521,17 @@ public:
     WC_D status_type insert(key_type key_in, const value_type& value_in, const tile<cg_size()>& group,
                             index_type probing_length = defaults::probing_length()) const noexcept {
         detail::ImmediateJoin join{status_};
-        return view().insert(key_in, value_in, group, probing_length, join);
+        return state().insert(key_in, value_in, group, probing_length, join);
     }
     WC_D status_type retrieve(key_type key_in, value_type& value_out, const tile<cg_size()>& group,
                               index_type probing_length = defaults::probing_length()) const noexcept {
         detail::ImmediateJoin join{status_};
-        return view().retrieve(key_in, value_out, group, probing_length, join);
+        return state().retrieve(key_in, value_out, group, probing_length, join);
     }
     WC_D status_type erase(key_type key_in, const tile<cg_size()>& group,
                            index_type probing_length = defaults::probing_length()) const noexcept {
         detail::ImmediateJoin join{status_};
-        return view().erase(key_in, group, probing_length, join);
+        return state().erase(key_in, group, probing_length, join);
     }
 
     // ------------------------------------------------------------- host API
@@ -533,9 +542,14 @@ public:
                      typename StatusHandler::base_type* status_out = nullptr) noexcept {
         static_assert(checks::is_status_handler<StatusHandler>(), "not a valid status handler type");
         if (!is_initialized_ || num_in == 0) return;
+        if constexpr (!soa_storage && detail::partition_capable<view_type>()) {
+            if (insert_partitioned<StatusHandler>(keys_in, values_in, num_in, stream, probing_length, status_out)) return;
+        } else {
+            mutations_.note(stream);
+        }
         if constexpr (soa_storage) {
             kernels::insert<view_type, StatusHandler><<<detail::grid_for(num_in, cg_size()), block_size(), 0, stream>>>(
-                keys_in, values_in, num_in, view(), probing_length, status_out);
+                keys_in, values_in, num_in, state(), probing_length, status_out);
         } else {
             insert_aos<StatusHandler>(keys_in, values_in, num_in, stream, probing_length, status_out);
         }
@@ -550,7 +564,7 @@ public:
         if (!is_initialized_ || num_in == 0) return;
         if constexpr (soa_storage) {
             kernels::retrieve<view_type, StatusHandler><<<detail::grid_for(num_in, cg_size()), block_size(), 0, stream>>>(
-                keys_in, num_in, values_out, view(), probing_length, status_out);
+                keys_in, num_in, values_out, state(), probing_length, status_out);
         } else {
             retrieve_aos<StatusHandler>(keys_in, num_in, values_out, stream, probing_length, status_out);
         }
@@ -563,7 +577,7 @@ public:
         index_type* tmp = temp_.get();
         (void)hipMemsetAsync(tmp, 0, sizeof(index_type), stream);
         kernels::retrieve_all<view_type>
-            <<<detail::grid_for(capacity(), 1, 8), block_size(), 0, stream>>>(keys_out, values_out, tmp, view());
+            <<<detail::grid_for(capacity(), 1, 8), block_size(), 0, stream>>>(keys_out, values_out, tmp, state());
         (void)hipMemcpyAsync(&num_out, tmp, sizeof(index_type), hipMemcpyDeviceToHost, stream);
         (void)hipStreamSynchronize(stream);
     }
@@ -575,22 +589,23 @@ public:
                     typename StatusHandler::base_type* status_out = nullptr) noexcept {
         static_assert(checks::is_status_handler<StatusHandler>(), "not a valid status handler type");
         if (!is_initialized_ || num_in == 0) return;
+        mutations_.note(stream);
         if constexpr (!soa_storage && detail::fixed_step_scheme<typename view_type::probing_scheme_type>::value) {
             if constexpr (detail::owner_capable<view_type>()) {
                 if (detail::owner_lookups()) {
-                    detail::launch_erase_owner<view_type, StatusHandler>(keys_in, num_in, view(), probing_length,
+                    detail::launch_erase_owner<view_type, StatusHandler>(keys_in, num_in, state(), probing_length,
                                                                          status_out, stream);
                     return;
                 }
             }
             if (detail::lockstep_lookups()) {
                 detail::launch_erase_lockstep<view_type, StatusHandler, detail::lockstep_keys<unsigned(cg_size())>()>(
-                    keys_in, num_in, view(), probing_length, status_out, stream);
+                    keys_in, num_in, state(), probing_length, status_out, stream);
                 return;
             }
         }
         kernels::erase<view_type, StatusHandler>
-            <<<detail::grid_for(num_in, cg_size()), block_size(), 0, stream>>>(keys_in, num_in, view(),
+            <<<detail::grid_for(num_in, cg_size()), block_size(), 0, stream>>>(keys_in, num_in, state(),
                                                                                 probing_length, status_out);
     }
 
@@ -599,7 +614,7 @@ public:
     WC_H void for_each(Func f, hipStream_t stream = 0, index_type smem_bytes = 0) const noexcept {
         if (!is_initialized_) return;
         kernels::for_each<Func, view_type>
-            <<<detail::grid_for(capacity(), 1, 8), block_size(), smem_bytes, stream>>>(f, view());
+            <<<detail::grid_for(capacity(), 1, 8), block_size(), smem_bytes, stream>>>(f, state());
     }
 
     // single_value_hash_table.cuh:534-592
@@ -608,7 +623,7 @@ public:
         index_type out = 0;
         index_type* tmp = temp_.get();
         (void)hipMemsetAsync(tmp, 0, sizeof(index_type), stream);
-        kernels::size<view_type><<<detail::grid_for(capacity(), 1, 8), block_size(), 0, stream>>>(tmp, view());
+        kernels::size<view_type><<<detail::grid_for(capacity(), 1, 8), block_size(), 0, stream>>>(tmp, state());
         (void)hipMemcpyAsync(&out, tmp, sizeof(index_type), hipMemcpyDeviceToHost, stream);
         (void)hipStreamSynchronize(stream);
         return out;
@@ -621,7 +636,7 @@ public:
         index_type out = 0;
         index_type* tmp = temp_.get();
         (void)hipMemsetAsync(tmp, 0, sizeof(index_type), stream);
-        kernels::size<view_type><<<detail::grid_for(capacity(), 1, 8), block_size(), 0, stream>>>(tmp, view(), true);
+        kernels::size<view_type><<<detail::grid_for(capacity(), 1, 8), block_size(), 0, stream>>>(tmp, state(), true);
         (void)hipMemcpyAsync(&out, tmp, sizeof(index_type), hipMemcpyDeviceToHost, stream);
         (void)hipStreamSynchronize(stream);
         return out;
@@ -663,6 +678,12 @@ public:
 
     // Device state handed to kernels.
     WC_HD view_type view() const noexcept {
+        mutations_.share();   // the holder may modify the table
+        return state();
+    }
+
+private:
+    WC_HD view_type state() const noexcept {
         if constexpr (soa_storage) {
             return view_type{table_.keys(), table_.values(), status_, geo_, seed_, is_initialized_};
         } else {
@@ -670,7 +691,33 @@ public:
         }
     }
 
-private:
+    // The partitioned insert of a batch that fills much of the table (see
+    // partition.hpp), where nothing else can modify the table meanwhile;
+    // advances the arguments past the keys it took, true if that is all.
+    template<class StatusHandler>
+    WC_H bool insert_partitioned(const key_type*& keys_in, const value_type*& values_in, index_type& num_in,
+                                 hipStream_t stream, index_type probing_length,
+                                 typename StatusHandler::base_type*& status_out) noexcept {
+        if (!detail::refill_inserts() || !detail::owner_inserts() ||
+            capacity() * sizeof(slot_type) <= detail::lane_insert_table_bytes() ||
+            !detail::partition_pays<view_type>(num_in, geo_)) {
+            mutations_.note(stream);
+            return false;
+        }
+        detail::MutationTracker::Exclusive exclusive(mutations_, stream);
+        if (!exclusive.granted()) return false;
+        const index_type done = detail::insert_partitioned<view_type, StatusHandler, true, slot_type>(
+            keys_in, values_in, num_in, state(), probing_length, status_out, stream);
+        if (done == 0) return false;
+        exclusive.use();
+        keys_in += done;
+        values_in += done;
+        num_in -= done;
+        if constexpr (!std::is_same<StatusHandler, status_handlers::ReturnNothing>::value)
+            if (status_out != nullptr) status_out += done;
+        return num_in == 0;
+    }
+
     // Bulk kernels of AoS tables: lane-per-key windows on small tables,
     // refill (default), lockstep or streaming cooperative kernels above.
     template<class StatusHandler>
@@ -680,7 +727,7 @@ private:
             if (capacity() * sizeof(slot_type) <= detail::lane_insert_table_bytes()) {
                 filter_valid_ = false;   // these kernels do not keep the overflow filter
                 kernels::insert_lanes<view_type, StatusHandler, detail::keys_per_lane(), true>
-                    <<<detail::grid_for_lanes(num_in), block_size(), 0, stream>>>(keys_in, values_in, num_in, view(),
+                    <<<detail::grid_for_lanes(num_in), block_size(), 0, stream>>>(keys_in, values_in, num_in, state(),
                                                                                  probing_length, status_out);
                 return;
             }
@@ -688,21 +735,21 @@ private:
         if constexpr (detail::fixed_step_scheme<typename view_type::probing_scheme_type>::value) {
             if (detail::refill_inserts()) {
                 detail::launch_insert_refill<view_type, StatusHandler, detail::refill_insert_keys<unsigned(cg_size())>(), true>(
-                    keys_in, values_in, num_in, view(), probing_length, status_out, stream);
+                    keys_in, values_in, num_in, state(), probing_length, status_out, stream);
                 return;
             }
             if (detail::lockstep_inserts()) {
                 filter_valid_ = false;
                 detail::launch_insert_lockstep<view_type, StatusHandler,
                                                detail::lockstep_insert_keys<unsigned(cg_size())>(), true>(
-                    keys_in, values_in, num_in, view(), probing_length, status_out, stream);
+                    keys_in, values_in, num_in, state(), probing_length, status_out, stream);
                 return;
             }
         }
         filter_valid_ = false;
         kernels::insert_batched<view_type, StatusHandler, detail::keys_per_group(), true>
             <<<detail::grid_for_batched(num_in, cg_size()), block_size(), 0, stream>>>(
-                keys_in, values_in, num_in, view(), probing_length, status_out);
+                keys_in, values_in, num_in, state(), probing_length, status_out);
     }
 
     template<class StatusHandler>
@@ -711,7 +758,7 @@ private:
         if constexpr (detail::LaneWindow<slot_type, cg_size()>::usable) {
             if (capacity() * sizeof(slot_type) <= detail::lane_table_bytes()) {
                 kernels::retrieve_lanes<view_type, StatusHandler, detail::keys_per_lane()>
-                    <<<detail::grid_for_lanes(num_in), block_size(), 0, stream>>>(keys_in, num_in, values_out, view(),
+                    <<<detail::grid_for_lanes(num_in), block_size(), 0, stream>>>(keys_in, num_in, values_out, state(),
                                                                                  probing_length, status_out);
                 return;
             }
@@ -719,18 +766,18 @@ private:
         if constexpr (detail::fixed_step_scheme<typename view_type::probing_scheme_type>::value) {
             if (detail::refill_lookups()) {
                 detail::launch_retrieve_refill<view_type, StatusHandler, detail::refill_keys<unsigned(cg_size())>()>(
-                    keys_in, num_in, values_out, view(), probing_length, status_out, stream);
+                    keys_in, num_in, values_out, state(), probing_length, status_out, stream);
                 return;
             }
             if (detail::lockstep_lookups()) {
                 detail::launch_retrieve_lockstep<view_type, StatusHandler, detail::lockstep_keys<unsigned(cg_size())>()>(
-                    keys_in, num_in, values_out, view(), probing_length, status_out, stream);
+                    keys_in, num_in, values_out, state(), probing_length, status_out, stream);
                 return;
             }
         }
         kernels::retrieve_batched<view_type, StatusHandler, detail::keys_per_group()>
             <<<detail::grid_for_batched(num_in, cg_size()), block_size(), 0, stream>>>(
-                keys_in, num_in, values_out, view(), probing_length, status_out);
+                keys_in, num_in, values_out, state(), probing_length, status_out);
     }
 
     WC_H void assign_status(status_type status, hipStream_t stream = 0) const noexcept {
@@ -768,6 +815,7 @@ private:
     // the filter holds every insert since init (cleared when an insert ran
     // on kernels that do not maintain it; lookups then ignore it)
     mutable bool filter_valid_ = false;
+    detail::MutationTracker mutations_;
 
     template<class K_, class V_, K_ E_, K_ T_, class P_, class S_, index_t B_> friend class CountingHashTable;
     template<class K_, class V_, K_ E_, K_ T_, class VS_, class P_> friend class BucketListHashTable;

@@ -1,0 +1,164 @@
+// Scratch memory of bulk calls, shared by all tables of the process.
+//
+// A bulk call leases one buffer for the kernels it launches. The lease ends
+// with the call; the buffer is handed out again at once, and its next user's
+// stream first waits (on the device) for the event recorded behind the last
+// user's kernels, so calls on one stream reuse one buffer and calls on
+// several streams or host threads get buffers of their own while the bound
+// allows. Bounded: at most kWorkspaceLimit bytes per device; a lease that
+// would exceed it, or that finds no device memory, is empty and the caller
+// runs its kernels that need no scratch. Given back: the buffers are freed
+// when the process's last table is destroyed, and idle ones before the bound
+// or the device's memory would refuse a larger lease.
+//
+// Not for calls under stream capture: a graph would keep the buffer's address
+// beyond the lease.
+#pragma once
+
+#include "base.hpp"
+
+#include <mutex>
+#include <vector>
+
+namespace warpcore {
+namespace detail {
+
+constexpr std::size_t kWorkspaceLimit = std::size_t(16) << 30;
+constexpr std::size_t kWorkspaceUnit = std::size_t(1) << 20;   // leases are rounded up to this
+
+class WorkspacePool {
+public:
+    static WorkspacePool& instance() noexcept {
+        static WorkspacePool* pool = new WorkspacePool;   // never destroyed: tables may outlive static objects
+        return *pool;
+    }
+
+    struct Buffer {
+        void* p = nullptr;
+        std::size_t bytes = 0;
+        int device = 0;
+        hipEvent_t done = nullptr;   // behind the last user's kernels
+        bool leased = false;
+    };
+
+    WC_H void add_user() noexcept {
+        std::lock_guard<std::mutex> lock(mu_);
+        ++users_;
+    }
+    WC_H void remove_user() noexcept {
+        std::lock_guard<std::mutex> lock(mu_);
+        if (--users_ == 0) free_idle(-1);
+    }
+
+    // a buffer of at least `bytes` on the current device, whose earlier use
+    // `stream` waits for; null without one
+    WC_H Buffer* acquire(std::size_t bytes, hipStream_t stream) noexcept {
+        bytes = (bytes + kWorkspaceUnit - 1) / kWorkspaceUnit * kWorkspaceUnit;
+        int device = 0;
+        if (bytes > kWorkspaceLimit || hipGetDevice(&device) != hipSuccess) return nullptr;
+        std::lock_guard<std::mutex> lock(mu_);
+        Buffer* best = nullptr;
+        for (Buffer* b : buffers_)
+            if (!b->leased && b->device == device && b->bytes >= bytes && (best == nullptr || b->bytes < best->bytes))
+                best = b;
+        if (best != nullptr) {
+            if (hipStreamWaitEvent(stream, best->done, 0) != hipSuccess) {
+                (void)hipGetLastError();
+                return nullptr;
+            }
+            best->leased = true;
+            return best;
+        }
+        std::size_t held = 0;
+        for (const Buffer* b : buffers_)
+            if (b->device == device) held += b->bytes;
+        if (held + bytes > kWorkspaceLimit) {
+            free_idle(device);
+            held = 0;
+            for (const Buffer* b : buffers_)
+                if (b->device == device) held += b->bytes;
+            if (held + bytes > kWorkspaceLimit) return nullptr;
+        }
+        Buffer* b = new (std::nothrow) Buffer;
+        if (b == nullptr) return nullptr;
+        b->bytes = bytes;
+        b->device = device;
+        if (hipEventCreateWithFlags(&b->done, hipEventDisableTiming) != hipSuccess) {
+            (void)hipGetLastError();
+            delete b;
+            return nullptr;
+        }
+        if (hipMalloc(&b->p, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            free_idle(device);
+            if (hipMalloc(&b->p, bytes) != hipSuccess) {
+                (void)hipGetLastError();
+                (void)hipEventDestroy(b->done);
+                delete b;
+                return nullptr;
+            }
+        }
+        b->leased = true;
+        buffers_.push_back(b);
+        return b;
+    }
+    WC_H void release(Buffer* b, hipStream_t stream) noexcept {
+        std::lock_guard<std::mutex> lock(mu_);
+        if (hipEventRecord(b->done, stream) != hipSuccess) {
+            (void)hipGetLastError();
+            (void)hipStreamSynchronize(stream);   // no event to wait for: the kernels end here
+        }
+        b->leased = false;
+        if (users_ == 0) free_idle(-1);
+    }
+    // bytes held on all devices
+    WC_H std::size_t bytes_held() noexcept {
+        std::lock_guard<std::mutex> lock(mu_);
+        std::size_t held = 0;
+        for (const Buffer* b : buffers_) held += b->bytes;
+        return held;
+    }
+
+private:
+    // frees the buffers not leased (of one device, or all); hipFree waits
+    // for the kernels that still use one
+    WC_H void free_idle(int device) noexcept {
+        std::size_t kept = 0;
+        for (Buffer* b : buffers_) {
+            if (b->leased || (device >= 0 && b->device != device)) {
+                buffers_[kept++] = b;
+                continue;
+            }
+            (void)hipEventSynchronize(b->done);
+            (void)hipFree(b->p);
+            (void)hipEventDestroy(b->done);
+            delete b;
+        }
+        buffers_.resize(kept);
+    }
+
+    std::mutex mu_;
+    std::vector<Buffer*> buffers_;
+    std::size_t users_ = 0;
+};
+
+// One bulk call's lease; false when the pool has no buffer for it.
+class WorkspaceLease {
+public:
+    WC_H WorkspaceLease(std::size_t bytes, hipStream_t stream) noexcept
+        : buffer_(WorkspacePool::instance().acquire(bytes, stream)), stream_(stream) {}
+    WorkspaceLease(const WorkspaceLease&) = delete;
+    WorkspaceLease& operator=(const WorkspaceLease&) = delete;
+    WC_H ~WorkspaceLease() noexcept {
+        if (buffer_ != nullptr) WorkspacePool::instance().release(buffer_, stream_);
+    }
+    explicit operator bool() const noexcept { return buffer_ != nullptr; }
+    void* get() const noexcept { return buffer_ != nullptr ? buffer_->p : nullptr; }
+
+private:
+    WorkspacePool::Buffer* buffer_;
+    hipStream_t stream_;
+};
+
+}  // namespace detail
+}  // namespace warpcore
