@@ -157,3 +157,78 @@ def test_inserts_from_two_streams(cuda):
         t.retrieve(kd, out, stream=a)
         torch.cuda.synchronize()
         assert torch.equal(out, vd)
+
+
+@pytest.mark.parametrize("kb,n,load,shape", [
+    (32, 1 << 20, 0.9, "distinct"), (32, 16_000_003, 0.9, "repeats"),   # one pass and two
+    (32, 3_000_001, 0.93, "hot"), (32, 16_000_003, 0.9, "few"),
+    (64, 1_500_001, 0.9, "invalid"), (64, 8_000_009, 0.9, "repeats"),
+])
+@pytest.mark.parametrize("statuses", [False, True])
+def test_set_insert(cuda, kb, n, load, shape, statuses):
+    from warpcore_amd.tables import HashSet
+    keys = _batch(n, kb, shape, seed=n)
+    h = HashSet(math.ceil(n / load), kb)
+    st = dev_empty(n, 32, 0x77)
+    h.insert(to_dev(keys), status_out=st if statuses else None)
+    valid = _valid(keys, kb)
+    uniq = np.unique(keys[valid])
+    assert h.size() == len(uniq)
+    word = (S_DUP if len(uniq) < valid.sum() else 0) | (S_INVALID_KEY if not valid.all() else 0)
+    assert int(h.pop_status()) == word
+    if statuses:
+        got = from_dev(st, np.uint32)
+        assert (got[~valid] == S_INVALID_KEY).all()
+        assert (_status_counts(keys, got, kb) == 1).all()
+    flags = torch.zeros(n, dtype=torch.uint8, device="cuda")
+    h.contains(to_dev(keys), flags)
+    assert bool((flags.cpu().numpy()[valid] == 1).all())
+    absent = unique_keys(100_000, kb, seed=3, exclude=uniq)
+    flags.fill_(7)
+    h.contains(to_dev(absent), flags[: len(absent)])
+    assert int(flags[: len(absent)].sum()) == 0
+
+
+@pytest.mark.parametrize("kb,n,distinct,skew", [
+    (64, 1 << 22, 1 << 20, 0.0), (64, 9_000_001, 3_700_000, 0.0), (64, 9_000_001, 3_700_000, 1.1),
+    (32, 6_000_003, 1_000_003, 0.7),
+])
+@pytest.mark.parametrize("statuses", [False, True])
+def test_counting_insert(cuda, kb, n, distinct, skew, statuses):
+    """Counts of two calls on top of each other, the second on keys half new."""
+    from warpcore_amd.tables import CountingHashTable
+    rng = np.random.default_rng(n)
+    uniq = unique_keys(distinct, kb, seed=n)
+    t = CountingHashTable(math.ceil(distinct / 0.85), kb)
+    total = np.zeros(distinct, np.int64)
+    for call in range(2):
+        hi = distinct // 2 if call == 0 else distinct
+        w = np.arange(1, hi + 1, dtype=np.float64) ** -skew
+        pick = np.searchsorted(np.cumsum(w / w.sum()), rng.random(n)).clip(max=hi - 1)
+        before = total > 0
+        total += np.bincount(pick, minlength=distinct)
+        st = dev_empty(n, 32, 0x77)
+        t.insert(to_dev(uniq[pick]), status_out=st if statuses else None)
+        if statuses:
+            got = from_dev(st, np.uint32)
+            assert set(np.unique(got)) <= {S_NONE, S_DUP}
+            none = np.bincount(pick, weights=(got == S_NONE), minlength=distinct)
+            np.testing.assert_array_equal(none, (total > 0) & ~before)
+    assert int(t.pop_status()) == S_DUP
+    assert t.size() == (total > 0).sum()
+    out, found = dev_empty(distinct, 64, 0), dev_empty(distinct, 32, 0x77)
+    t.retrieve(to_dev(uniq), out, status_out=found)
+    np.testing.assert_array_equal(from_dev(out, np.int64) * (total > 0), total)
+    np.testing.assert_array_equal(from_dev(found, np.uint32) == S_NONE, total > 0)
+
+
+def test_counting_with_maximum(cuda):
+    """A maximum count: the general insert, which stops there."""
+    from warpcore_amd.tables import CountingHashTable
+    uniq = unique_keys(1 << 20, 64, seed=4)
+    keys = np.tile(uniq, 5)
+    t = CountingHashTable(1 << 21, 64, max_count=3)
+    t.insert(to_dev(keys))
+    out = dev_empty(len(uniq), 64, 0)
+    t.retrieve(to_dev(uniq), out)
+    assert (from_dev(out, np.uint64) == 3).all()

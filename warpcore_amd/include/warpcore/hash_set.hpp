@@ -41,6 +41,7 @@ struct HashSetView {
     using out_type = bool;
     using probe_slot_type = Key;
     static constexpr bool publishes_value = false;
+    static constexpr RegionOp region_op = RegionOp::none;   // partitioned inserts (partition.hpp)
     WC_HD bool ready() const noexcept { return initialized; }
     WC_HD Key hash_seed() const noexcept { return seed; }
     WC_HD const probing_schemes::Geometry& geometry() const noexcept { return geo; }
@@ -165,6 +166,7 @@ public:
           capacity_(detail::get_valid_capacity(min_capacity, cg_size())),
           temp_(TempMemoryBytes / sizeof(index_type)), seed_(seed), is_initialized_(false), is_copy_(false),
           geo_(probing_schemes::Geometry::make(capacity_, cg_size())) {
+        detail::WorkspacePool::instance().add_user();
         const std::size_t bytes = sizeof(key_type) * capacity_;
         if (hipMalloc(&status_, sizeof(status_type)) != hipSuccess) { status_ = nullptr; return; }
         if (capacity_ == 0) { assign_status(Status::invalid_configuration() + Status::not_initialized()); return; }
@@ -179,10 +181,11 @@ public:
     }
     WC_HD HashSet(const HashSet& o) noexcept
         : status_(o.status_), keys_(o.keys_), capacity_(o.capacity_), temp_(o.temp_), seed_(o.seed_),
-          is_initialized_(o.is_initialized_), is_copy_(true), geo_(o.geo_) {}
+          is_initialized_(o.is_initialized_), is_copy_(true), geo_(o.geo_), mutations_(o.mutations_) {}
     WC_H HashSet(HashSet&& o) noexcept
         : status_(o.status_), keys_(o.keys_), capacity_(o.capacity_), temp_(std::move(o.temp_)), seed_(o.seed_),
-          is_initialized_(o.is_initialized_), is_copy_(o.is_copy_), geo_(o.geo_) {
+          is_initialized_(o.is_initialized_), is_copy_(o.is_copy_), geo_(o.geo_),
+          mutations_(std::move(o.mutations_)) {
         o.is_copy_ = true;
     }
     WC_HD ~HashSet() noexcept {
@@ -190,6 +193,8 @@ public:
         if (!is_copy_) {
             if (keys_ != nullptr) (void)hipFree(keys_);
             if (status_ != nullptr) (void)hipFree(status_);
+            mutations_.destroy();
+            detail::WorkspacePool::instance().remove_user();
         }
 #endif
     }
@@ -197,6 +202,7 @@ public:
     // hash_set.cuh:142-161
     WC_H void init(key_type seed, hipStream_t stream = 0) noexcept {
         seed_ = seed;
+        mutations_.restart();
         if (is_initialized_) {
             kernels::memset<key_type><<<detail::grid_for(capacity_, 1, 8), block_size(), 0, stream>>>(
                 keys_, capacity_, empty_key());
@@ -208,17 +214,17 @@ public:
     WC_D status_type insert(key_type key_in, const tile<cg_size()>& group,
                             index_type probing_length = defaults::probing_length()) const noexcept {
         detail::ImmediateJoin join{status_};
-        return view().insert(key_in, group, probing_length, join);
+        return state().insert(key_in, group, probing_length, join);
     }
     WC_D status_type retrieve(key_type key_in, bool& flag_out, const tile<cg_size()>& group,
                               index_type probing_length = defaults::probing_length()) const noexcept {
         detail::ImmediateJoin join{status_};
-        return view().retrieve(key_in, flag_out, group, probing_length, join);
+        return state().retrieve(key_in, flag_out, group, probing_length, join);
     }
     WC_D status_type erase(key_type key_in, const tile<cg_size()>& group,
                            index_type probing_length = defaults::probing_length()) const noexcept {
         detail::ImmediateJoin join{status_};
-        return view().erase(key_in, group, probing_length, join);
+        return state().erase(key_in, group, probing_length, join);
     }
 
     template<class StatusHandler = defaults::status_handler_t>
@@ -227,10 +233,19 @@ public:
                      typename StatusHandler::base_type* status_out = nullptr) noexcept {
         static_assert(checks::is_status_handler<StatusHandler>(), "not a valid status handler type");
         if (!is_initialized_ || num_in == 0) return;
+        if constexpr (detail::partition_capable<view_type>()) {
+            const bool* values = nullptr;
+            if (detail::insert_partitioned_first<view_type, StatusHandler, false, key_type>(
+                    mutations_, keys_in, values, num_in, state(), probing_length, status_out, stream,
+                    capacity() * sizeof(key_type)))
+                return;
+        } else {
+            mutations_.note(stream);
+        }
         if constexpr (detail::LaneWindow<key_type, cg_size()>::usable) {
             if (capacity() * sizeof(key_type) <= detail::lane_insert_table_bytes()) {
                 kernels::insert_lanes<view_type, StatusHandler, detail::keys_per_lane(), false>
-                    <<<detail::grid_for_lanes(num_in), block_size(), 0, stream>>>(keys_in, nullptr, num_in, view(),
+                    <<<detail::grid_for_lanes(num_in), block_size(), 0, stream>>>(keys_in, nullptr, num_in, state(),
                                                                                  probing_length, status_out);
                 return;
             }
@@ -238,19 +253,19 @@ public:
         if constexpr (detail::fixed_step_scheme<typename view_type::probing_scheme_type>::value) {
             if (detail::refill_inserts()) {
                 detail::launch_insert_refill<view_type, StatusHandler, detail::refill_insert_keys<unsigned(cg_size())>(), false>(
-                    keys_in, nullptr, num_in, view(), probing_length, status_out, stream);
+                    keys_in, nullptr, num_in, state(), probing_length, status_out, stream);
                 return;
             }
             if (detail::lockstep_inserts()) {
                 detail::launch_insert_lockstep<view_type, StatusHandler,
                                                detail::lockstep_insert_keys<unsigned(cg_size())>(), false>(
-                    keys_in, nullptr, num_in, view(), probing_length, status_out, stream);
+                    keys_in, nullptr, num_in, state(), probing_length, status_out, stream);
                 return;
             }
         }
         kernels::insert_batched<view_type, StatusHandler, detail::keys_per_group(), false>
             <<<detail::grid_for_batched(num_in, cg_size()), block_size(), 0, stream>>>(
-                keys_in, nullptr, num_in, view(), probing_length, status_out);
+                keys_in, nullptr, num_in, state(), probing_length, status_out);
     }
 
     // membership per key; flags_out[i] is written when status_out[i] is none
@@ -263,7 +278,7 @@ public:
         if constexpr (detail::LaneWindow<key_type, cg_size()>::usable) {
             if (capacity() * sizeof(key_type) <= detail::lane_table_bytes()) {
                 kernels::retrieve_lanes<view_type, StatusHandler, detail::keys_per_lane()>
-                    <<<detail::grid_for_lanes(num_in), block_size(), 0, stream>>>(keys_in, num_in, flags_out, view(),
+                    <<<detail::grid_for_lanes(num_in), block_size(), 0, stream>>>(keys_in, num_in, flags_out, state(),
                                                                                  probing_length, status_out);
                 return;
             }
@@ -271,18 +286,18 @@ public:
         if constexpr (detail::fixed_step_scheme<typename view_type::probing_scheme_type>::value) {
             if (detail::refill_lookups()) {
                 detail::launch_retrieve_refill<view_type, StatusHandler, detail::refill_keys<unsigned(cg_size())>()>(
-                    keys_in, num_in, flags_out, view(), probing_length, status_out, stream);
+                    keys_in, num_in, flags_out, state(), probing_length, status_out, stream);
                 return;
             }
             if (detail::lockstep_lookups()) {
                 detail::launch_retrieve_lockstep<view_type, StatusHandler, detail::lockstep_keys<unsigned(cg_size())>()>(
-                    keys_in, num_in, flags_out, view(), probing_length, status_out, stream);
+                    keys_in, num_in, flags_out, state(), probing_length, status_out, stream);
                 return;
             }
         }
         kernels::retrieve_batched<view_type, StatusHandler, detail::keys_per_group()>
             <<<detail::grid_for_batched(num_in, cg_size()), block_size(), 0, stream>>>(
-                keys_in, num_in, flags_out, view(), probing_length, status_out);
+                keys_in, num_in, flags_out, state(), probing_length, status_out);
     }
     template<class StatusHandler = defaults::status_handler_t>
     WC_H void contains(const key_type* keys_in, index_type num_in, bool* flags_out, hipStream_t stream = 0,
@@ -297,7 +312,7 @@ public:
         index_type* tmp = temp_.get();
         (void)hipMemsetAsync(tmp, 0, sizeof(index_type), stream);
         kernels::retrieve_all<view_type>
-            <<<detail::grid_for(capacity(), 1, 8), block_size(), 0, stream>>>(keys_out, nullptr, tmp, view());
+            <<<detail::grid_for(capacity(), 1, 8), block_size(), 0, stream>>>(keys_out, nullptr, tmp, state());
         (void)hipMemcpyAsync(&num_out, tmp, sizeof(index_type), hipMemcpyDeviceToHost, stream);
         (void)hipStreamSynchronize(stream);
     }
@@ -307,8 +322,9 @@ public:
                     index_type probing_length = defaults::probing_length(),
                     typename StatusHandler::base_type* status_out = nullptr) noexcept {
         if (!is_initialized_ || num_in == 0) return;
+        mutations_.note(stream);
         kernels::erase<view_type, StatusHandler>
-            <<<detail::grid_for(num_in, cg_size()), block_size(), 0, stream>>>(keys_in, num_in, view(),
+            <<<detail::grid_for(num_in, cg_size()), block_size(), 0, stream>>>(keys_in, num_in, state(),
                                                                                 probing_length, status_out);
     }
 
@@ -316,7 +332,7 @@ public:
     WC_H void for_each(Func f, hipStream_t stream = 0, index_type smem_bytes = 0) const noexcept {
         if (!is_initialized_) return;
         kernels::for_each_key<Func, view_type>
-            <<<detail::grid_for(capacity(), 1, 8), block_size(), smem_bytes, stream>>>(f, view());
+            <<<detail::grid_for(capacity(), 1, 8), block_size(), smem_bytes, stream>>>(f, state());
     }
 
     WC_H index_type size(hipStream_t stream = 0) const noexcept {
@@ -324,7 +340,7 @@ public:
         index_type out = 0;
         index_type* tmp = temp_.get();
         (void)hipMemsetAsync(tmp, 0, sizeof(index_type), stream);
-        kernels::size<view_type><<<detail::grid_for(capacity(), 1, 8), block_size(), 0, stream>>>(tmp, view());
+        kernels::size<view_type><<<detail::grid_for(capacity(), 1, 8), block_size(), 0, stream>>>(tmp, state());
         (void)hipMemcpyAsync(&out, tmp, sizeof(index_type), hipMemcpyDeviceToHost, stream);
         (void)hipStreamSynchronize(stream);
         return out;
@@ -358,9 +374,13 @@ public:
     }
     WC_HD key_type seed() const noexcept { return seed_; }
     WC_HD bool is_copy() const noexcept { return is_copy_; }
-    WC_HD view_type view() const noexcept { return view_type{keys_, status_, geo_, seed_, is_initialized_}; }
+    WC_HD view_type view() const noexcept {
+        mutations_.share();   // the holder may modify the set
+        return state();
+    }
 
 private:
+    WC_HD view_type state() const noexcept { return view_type{keys_, status_, geo_, seed_, is_initialized_}; }
     WC_H void assign_status(status_type status, hipStream_t stream = 0) const noexcept {
         if (status_ != nullptr) {
             (void)hipMemcpyAsync(status_, &status, sizeof(status_type), hipMemcpyHostToDevice, stream);
@@ -376,6 +396,7 @@ private:
     bool is_initialized_;
     bool is_copy_;
     probing_schemes::Geometry geo_;
+    detail::MutationTracker mutations_;
 };
 
 }  // namespace warpcore

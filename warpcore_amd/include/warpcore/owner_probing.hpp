@@ -103,15 +103,16 @@ struct ArrayInput {
         else return V{};
     }
     WC_D static index_t position(index_t i) noexcept { return i; }
+    static constexpr bool skip_first = false;
 };
 
 // Inserts of keys first .. end of `in` by the calling wavefront (all 64 lanes
 // call this with the same range). `lds` holds 64 entries of this wave.
-// SkipFirst: every key's first window is known to be full, not to hold the
-// key, and marked in the overflow filter; its walk starts at the second
+// in.skip_first: every key's first window is known to be full, not to hold
+// the key, and marked in the overflow filter; its walk starts at the second
 // window (single-value cores: a multi-value core counts the key's values in
 // every window).
-template<class Core, class StatusHandler, class W, bool HasValues, unsigned SPL, bool SkipFirst, class Input>
+template<class Core, class StatusHandler, class W, bool HasValues, unsigned SPL, class Input>
 WC_D void insert_owner_from(const Input& in, index_t first, index_t end, const Core& core, index_t budget,
                             typename StatusHandler::base_type* __restrict__ status_out,
                             OwnerEntry<typename Core::key_type, W>* lds, DeferredJoin& join) {
@@ -125,7 +126,6 @@ WC_D void insert_owner_from(const Input& in, index_t first, index_t end, const C
     constexpr unsigned CG = WIN / SPL;                     // lanes per group
     static_assert(CG >= 2 && CG <= 64 && (CG & (CG - 1)) == 0, "groups of 2..64 lanes");
     constexpr bool multi = is_multi_value_core<Core>::value;
-    static_assert(!(multi && SkipFirst), "multi-value walks start at the first window");
     static_assert(SPL == 1 || (SPL == 2 && !multi && sizeof(Probe) == 8 && !std::is_same<Probe, K>::value),
                   "two slots per lane: packed 8-byte slots of single-value cores");
     constexpr bool keep_seen = !std::is_same<Probe, K>::value;
@@ -199,7 +199,7 @@ WC_D void insert_owner_from(const Input& in, index_t first, index_t end, const C
                 rnd = 0;
                 count = 0;
                 phase = kLoad;
-                if constexpr (SkipFirst) {
+                if (!multi && in.skip_first) {
                     if (budget <= 1) {
                         join(Status::probing_length_exceeded());
                         StatusHandler::handle(Status::probing_length_exceeded(), status_out, in.position(pos));
@@ -363,8 +363,7 @@ WC_D void insert_owner_range(const typename Core::key_type* __restrict__ keys_in
                              typename StatusHandler::base_type* __restrict__ status_out,
                              OwnerEntry<typename Core::key_type, W>* lds, DeferredJoin& join) {
     const ArrayInput<typename Core::key_type, typename Core::value_type, HasValues> in{keys_in, values_in};
-    insert_owner_from<Core, StatusHandler, W, HasValues, SPL, false>(in, first, end, core, budget, status_out, lds,
-                                                                     join);
+    insert_owner_from<Core, StatusHandler, W, HasValues, SPL>(in, first, end, core, budget, status_out, lds, join);
 }
 
 // Lookups of keys_in[first .. end) by the calling wavefront. A hit is

@@ -50,6 +50,7 @@
 #include "base.hpp"
 #include "batched_probing.hpp"
 #include "engine.hpp"
+#include "mutation.hpp"
 #include "owner_probing.hpp"
 #include "refill_probing.hpp"
 #include "status.hpp"
@@ -82,6 +83,12 @@ constexpr unsigned part_items() noexcept {   // records per thread of a tile
     return sizeof(Rec) >= 16 ? 4 : sizeof(Rec) >= 8 || Idx ? 8 : 16;
 }
 
+// Wavefronts per SIMD of the sorting kernels: their tiles leave LDS for two
+// blocks per CU with 16-byte records (8 wavefronts per SIMD, 64 VGPRs), else
+// for one.
+template<class Rec, bool Idx>
+constexpr unsigned part_waves() noexcept { return sizeof(Rec) >= 16 && !Idx ? 8 : 4; }
+
 // Windows per region: a power of two whose keys and values fill kRegionBytes.
 template<class Core>
 constexpr unsigned region_windows() noexcept {
@@ -91,6 +98,14 @@ constexpr unsigned region_windows() noexcept {
     while (2 * w * Core::cg_size() * per <= kRegionBytes) w *= 2;
     return w;
 }
+
+// Records a region's segment holds beyond a uniformly hashed batch's share.
+// Counters: the entries of one combining pass repeat keys that are frequent
+// but not frequent enough for its block maps, up to some 10^4 times (2^28
+// occurrences, Zipf 1.1: without the room those entries took the general
+// insert, 5.6 of 13.6 ms).
+template<class Core>
+constexpr unsigned region_slack() noexcept { return Core::region_op == RegionOp::add ? 32768 : 0; }
 
 // Shape of one run of the passes over at most n keys.
 struct PartPlan {
@@ -144,7 +159,7 @@ WC_H PartPlan make_part_plan(index_t n, const probing_schemes::Geometry& geo) no
     const index_t a_records = index_t(p.buckets) * kPartXcds * p.cap1;
     index_t b_records;
     if (p.two_pass()) {
-        p.cap2 = part_capacity(double(n) * std::min(1.0, per_region));
+        p.cap2 = part_capacity(double(n) * std::min(1.0, per_region)) + region_slack<Core>();
         p.tiles = unsigned(SDIV(index_t(p.cap1), index_t(p.tile)));
         const index_t bucket_bytes = (index_t(1) << p.p2log) * p.cap2 * rec;
         index_t gb = kRefineBytes / bucket_bytes / kPartXcds * kPartXcds;   // every XCD gets as many buckets
@@ -184,30 +199,46 @@ WC_D auto rec_key(const Rec& r) noexcept {
     else return r.key;
 }
 
-// Inputs of the lane-owner insert beside plain arrays: records (status
-// positions in idx, if any), and a list of positions of the batch.
-template<class K, class V, class Rec>
-struct RecordInput {
-    const Rec* rec;
-    const std::uint32_t* idx;
-    WC_D K key(index_t i) const noexcept { return rec_key(rec[i]); }
-    WC_D V value(index_t i) const noexcept {
-        if constexpr (std::is_integral<Rec>::value) return V{};
-        else return rec[i].value;
+// Input of the general inserts here, the same for the whole wavefront: the
+// batch, a list of its positions, or records, as keys and values at equal
+// distances.
+template<class K, class V, class Rec, bool HasValues>
+struct PartInput {
+    const unsigned char* keys;
+    const unsigned char* values;
+    std::uint32_t key_step, value_step;
+    const std::uint32_t* list;      // positions of the batch, or null
+    const std::uint32_t* where;     // positions of the records, or null
+    bool skip_first;
+    WC_D static PartInput records(const Rec* rec, const std::uint32_t* idx, bool skip) noexcept {
+        PartInput in;
+        in.keys = reinterpret_cast<const unsigned char*>(rec);
+        in.values = in.keys;
+        if constexpr (HasValues) in.values = reinterpret_cast<const unsigned char*>(&rec->value);
+        in.key_step = in.value_step = sizeof(Rec);
+        in.list = nullptr;
+        in.where = idx;
+        in.skip_first = skip;
+        return in;
     }
-    WC_D index_t position(index_t i) const noexcept { return idx != nullptr ? index_t(idx[i]) : i; }
-};
-template<class K, class V, bool HasValues>
-struct ListedInput {
-    const std::uint32_t* list;
-    const K* keys;
-    const V* values;
-    WC_D K key(index_t i) const noexcept { return keys[list[i]]; }
+    WC_D static PartInput batch(const K* keys, const V* values, const std::uint32_t* list) noexcept {
+        PartInput in;
+        in.keys = reinterpret_cast<const unsigned char*>(keys);
+        in.values = reinterpret_cast<const unsigned char*>(values);
+        in.key_step = sizeof(K);
+        in.value_step = sizeof(V);
+        in.list = list;
+        in.where = list;
+        in.skip_first = false;
+        return in;
+    }
+    WC_D index_t at(index_t i) const noexcept { return list != nullptr ? index_t(list[i]) : i; }
+    WC_D K key(index_t i) const noexcept { return *reinterpret_cast<const K*>(keys + at(i) * key_step); }
     WC_D V value(index_t i) const noexcept {
-        if constexpr (HasValues) return values[list[i]];
+        if constexpr (HasValues) return *reinterpret_cast<const V*>(values + at(i) * value_step);
         else return V{};
     }
-    WC_D index_t position(index_t i) const noexcept { return list[i]; }
+    WC_D index_t position(index_t i) const noexcept { return where != nullptr ? index_t(where[i]) : i; }
 };
 
 // Slots per lane of the general inserts here (as the lane-owner launches choose).
@@ -340,17 +371,14 @@ struct TileSort {
 
 namespace kernels {
 
-// Two blocks of 1024 threads per CU need 8 wavefronts per SIMD: 64 VGPRs.
-#define WC_PART_OCCUPANCY __attribute__((amdgpu_waves_per_eu(8)))
-
 // Clears the counters; the last block samples the batch: kPartSample keys at
 // equal distances, counted per key in LDS. *skewed = 1 when one of them came
-// kPartRepeat times (about one key in a thousand of the batch).
+// kPartRepeat times (about one key in a thousand of the batch); without
+// `sample` it is 0.
 template<class Core>
 __global__ __launch_bounds__(1024) void part_begin(std::uint32_t* __restrict__ counters, index_t num_counters,
                                                    const typename Core::key_type* __restrict__ keys_in, index_t num_in,
-                                                   const index_t* __restrict__ num_dev,
-                                                   std::uint32_t* __restrict__ skewed) {
+                                                   bool sample, std::uint32_t* __restrict__ skewed) {
     using K = typename Core::key_type;
     if (blockIdx.x + 1 < gridDim.x) {
         const index_t stride = index_t(gridDim.x - 1) * blockDim.x;
@@ -367,7 +395,7 @@ __global__ __launch_bounds__(1024) void part_begin(std::uint32_t* __restrict__ c
         scount[s] = 0;
     }
     if (threadIdx.x == 0) most = 0;
-    if (num_dev != nullptr && *num_dev < num_in) num_in = *num_dev;
+    if (!sample) num_in = 0;
     const index_t step = num_in / detail::kPartSample;
     constexpr unsigned P = detail::kPartSample / detail::kPartThreads;
     K key[P];
@@ -396,7 +424,7 @@ __global__ __launch_bounds__(1024) void part_begin(std::uint32_t* __restrict__ c
 // status starts as none (or invalid_key); later passes write the others.
 // 80 KB of LDS (16-byte records): two blocks per CU.
 template<class Core, class StatusHandler, class Rec, bool HasValues, bool Idx>
-__global__ __launch_bounds__(1024) WC_PART_OCCUPANCY void part_scatter(const typename Core::key_type* __restrict__ keys_in,
+__global__ __launch_bounds__(1024, (detail::part_waves<Rec, Idx>())) void part_scatter(const typename Core::key_type* __restrict__ keys_in,
                                                      const typename Core::value_type* __restrict__ values_in,
                                                      index_t num_in, const index_t* __restrict__ num_dev,
                                                      const std::uint32_t* __restrict__ skewed, Core core,
@@ -466,7 +494,7 @@ __global__ __launch_bounds__(1024) WC_PART_OCCUPANCY void part_scatter(const typ
 // cap2 ..] (R regions per bucket). A tile's records without room are left at
 // the tile's start, their number in left[].
 template<class Core, class Rec, bool Idx>
-__global__ __launch_bounds__(1024) WC_PART_OCCUPANCY void part_refine(Rec* __restrict__ in, std::uint32_t* __restrict__ in_idx,
+__global__ __launch_bounds__(1024, (detail::part_waves<Rec, Idx>())) void part_refine(Rec* __restrict__ in, std::uint32_t* __restrict__ in_idx,
                                                     const std::uint32_t* __restrict__ counts_in, Core core,
                                                     detail::PartPlan plan, unsigned first_bucket, unsigned last_bucket,
                                                     Rec* __restrict__ out, std::uint32_t* __restrict__ out_idx,
@@ -533,7 +561,7 @@ __global__ __launch_bounds__(256) void part_leftover(const Rec* __restrict__ rec
                                                      typename StatusHandler::base_type* __restrict__ status_out) {
     using K = typename Core::key_type;
     using V = typename Core::value_type;
-    using Input = detail::RecordInput<K, V, Rec>;
+    using Input = detail::PartInput<K, V, Rec, HasValues>;
     __shared__ detail::OwnerEntry<K, std::uint32_t> lds[256];
     detail::DeferredJoin join;
     const index_t budget = probing_schemes::detail::window_budget(probing_length, Core::cg_size(),
@@ -549,8 +577,8 @@ __global__ __launch_bounds__(256) void part_leftover(const Rec* __restrict__ rec
             const index_t unit = u + at;
             const index_t n = unsigned(__builtin_amdgcn_readlane(int(l), int(at)));
             const index_t base = unit / plan.tiles * plan.cap1 + unit % plan.tiles * plan.tile;
-            const Input in{rec + base, Idx ? rec_idx + base : nullptr};
-            detail::insert_owner_from<Core, StatusHandler, std::uint32_t, HasValues, detail::part_spl<Core>(), false>(
+            const Input in = Input::records(rec + base, Idx ? rec_idx + base : nullptr, false);
+            detail::insert_owner_from<Core, StatusHandler, std::uint32_t, HasValues, detail::part_spl<Core>()>(
                 in, 0, n, core, budget, status_out, lds + (threadIdx.x & ~63u), join);
         }
     }
@@ -565,7 +593,7 @@ __global__ __launch_bounds__(256) void part_leftover(const Rec* __restrict__ rec
 // two blocks per CU, so that one block's loads run beside the other's
 // probing.
 template<class Core, class StatusHandler, class Rec, unsigned Segments, bool HasValues, bool Idx>
-__global__ __launch_bounds__(1024) WC_PART_OCCUPANCY void part_build(const Rec* __restrict__ in, const std::uint32_t* __restrict__ in_idx,
+__global__ __launch_bounds__(1024, 8) void part_build(const Rec* __restrict__ in, const std::uint32_t* __restrict__ in_idx,
                                                    const std::uint32_t* __restrict__ counts, unsigned count_stride,
                                                    unsigned cap, unsigned first_region, unsigned last_region,
                                                    Core core, Rec* __restrict__ over_out,
@@ -584,7 +612,7 @@ __global__ __launch_bounds__(1024) WC_PART_OCCUPANCY void part_build(const Rec* 
     constexpr RegionOp op = Core::region_op;
     constexpr bool values = op != RegionOp::none;
     constexpr bool filtered = detail::has_overflow_filter<Core>::value;
-    constexpr unsigned I = sizeof(Rec) >= 16 ? 4 : 8;   // records per thread and round
+    constexpr unsigned I = sizeof(K) >= 8 || Idx ? 4 : 8;   // records per thread and round
     __shared__ alignas(16) K lkey[S];
     __shared__ V lval[values ? S : 1];
     __shared__ std::uint32_t lfilter[filtered ? RW / 4 : 1];
@@ -759,7 +787,7 @@ __global__ __launch_bounds__(256) void part_tail(const Rec* __restrict__ over, c
                                                  typename StatusHandler::base_type* __restrict__ status_out) {
     using K = typename Core::key_type;
     using V = typename Core::value_type;
-    using Input = detail::RecordInput<K, V, Rec>;
+    using Input = detail::PartInput<K, V, Rec, HasValues>;
     __shared__ detail::OwnerEntry<K, std::uint32_t> lds[256];
     auto* my = lds + (threadIdx.x & ~63u);
     detail::DeferredJoin join;
@@ -767,46 +795,36 @@ __global__ __launch_bounds__(256) void part_tail(const Rec* __restrict__ over, c
                                                                   core.geometry().windows);
     const index_t wave = (index_t(blockIdx.x) * blockDim.x + threadIdx.x) / 64;
     const index_t waves = (index_t(gridDim.x) * blockDim.x) / 64;
-    if (*skewed != 0) {
-        if (num_dev != nullptr && *num_dev < num_in) num_in = *num_dev;
-        index_t each = SDIV(num_in, waves);
-        each = each < 64 ? 64 : each;
-        const index_t lo = wave * each < num_in ? wave * each : num_in;
-        const index_t hi = lo + each < num_in ? lo + each : num_in;
-        const detail::ArrayInput<K, V, HasValues> in{keys_in, values_in};
-        detail::insert_owner_from<Core, StatusHandler, std::uint32_t, HasValues, detail::part_spl<Core>(), false>(
-            in, lo, hi, core, budget, status_out, my, join);
-        join.flush(core.status_word());
-        return;
-    }
-    index_t total = 0;
-    for (unsigned g = 0; g < groups; ++g) total += over_counts[g];
-    // shares of at least one key per lane
-    index_t per = SDIV(total, waves);
-    per = per < 64 ? 64 : per;
-    const index_t first = wave * per;
-    const index_t end = first + per < total ? first + per : total;
-    index_t base = 0;
-    for (unsigned g = 0; g < groups && base < end; ++g) {
-        const index_t n = over_counts[g];
-        const index_t lo = first > base ? first - base : 0;
-        const index_t hi = end - base < n ? end - base : n;
-        if (first < end && lo < hi) {
-            const Input in{over + g * stride, Idx ? over_idx + g * stride : nullptr};
-            detail::insert_owner_from<Core, StatusHandler, std::uint32_t, HasValues, detail::part_spl<Core>(), true>(
-                in, lo, hi, core, budget, status_out, my, join);
+    if (num_dev != nullptr && *num_dev < num_in) num_in = *num_dev;
+    const bool whole = *skewed != 0;
+    // part 0: the overflow lists, one after another; part 1: the listed
+    // positions of the batch, or (skewed) all of it. One call for both keeps
+    // the kernel to one copy of the insert.
+    const index_t listed = whole ? num_in : *spill_count;
+    index_t overflowed = 0;
+    if (!whole)
+        for (unsigned g = 0; g < groups; ++g) overflowed += over_counts[g];
+    for (unsigned part = 0; part < 2; ++part) {
+        // equal shares of at least one key per lane
+        const index_t total = part == 0 ? overflowed : listed;
+        index_t per = SDIV(total, waves);
+        per = per < 64 ? 64 : per;
+        const index_t first = wave * per;
+        const index_t end = first + per < total ? first + per : total;
+        const unsigned lists = part == 0 ? groups : 1;
+        index_t base = 0;
+        for (unsigned g = 0; g < lists; ++g) {
+            const index_t n = part == 0 ? over_counts[g] : total;
+            const index_t lo = first > base ? first - base : 0;
+            const index_t hi = end > base ? (end - base < n ? end - base : n) : 0;
+            Input in = Input::batch(keys_in, values_in, whole ? nullptr : spill_list);
+            if (part == 0)
+                in = Input::records(over + g * stride, Idx ? over_idx + g * stride : nullptr, true);
+            if (first < end && lo < hi)
+                detail::insert_owner_from<Core, StatusHandler, std::uint32_t, HasValues, detail::part_spl<Core>()>(
+                    in, lo, hi, core, budget, status_out, my, join);
+            base += n;
         }
-        base += n;
-    }
-    const index_t spilled = *spill_count;
-    if (spilled != 0) {
-        index_t each = SDIV(spilled, waves);
-        each = each < 64 ? 64 : each;
-        const index_t lo = wave * each < spilled ? wave * each : spilled;
-        const index_t hi = lo + each < spilled ? lo + each : spilled;
-        const detail::ListedInput<K, V, HasValues> in{spill_list, keys_in, values_in};
-        detail::insert_owner_from<Core, StatusHandler, std::uint32_t, HasValues, detail::part_spl<Core>(), false>(in, lo, hi, core, budget,
-                                                                                          status_out, my, join);
     }
     join.flush(core.status_word());
 }
@@ -858,7 +876,8 @@ WC_H bool partition_pays(index_t n, const probing_schemes::Geometry& geo) noexce
 }
 
 // Runs the passes over one chunk; false (nothing launched) without a
-// workspace for it.
+// workspace for it. With num_dev the chunk holds min(n, *num_dev) keys (a
+// count made on the device), none of them frequent, so none are sampled.
 template<class Core, class StatusHandler, bool HasValues, class Rec>
 WC_H bool insert_partitioned_chunk(const typename Core::key_type* keys_in, const typename Core::value_type* values_in,
                                    index_t n, const index_t* num_dev, const Core& core, index_t probing_length,
@@ -879,7 +898,7 @@ WC_H bool insert_partitioned_chunk(const typename Core::key_type* keys_in, const
     const std::uint32_t* skewed = word(p.skewed);
     const index_t clear = SDIV(p.counter_words, index_t(4 * kPartThreads));
     kernels::part_begin<Core><<<unsigned(clear < 256 ? clear : 256) + 1, kPartThreads, 0, stream>>>(
-        word(p.c1), p.counter_words, keys_in, n, num_dev, word(p.skewed));
+        word(p.c1), p.counter_words, keys_in, n, num_dev == nullptr, word(p.skewed));
     const index_t tiles = SDIV(n, index_t(p.tile));
     constexpr auto scatter = kernels::part_scatter<Core, StatusHandler, Rec, HasValues, Idx>;
     scatter<<<part_grid<scatter>(tiles), kPartThreads, 0, stream>>>(
@@ -934,6 +953,35 @@ WC_H index_t insert_partitioned(const typename Core::key_type* keys_in, const ty
         done += m;
     }
     return done;
+}
+
+// The partitioned insert of a batch that fills much of the table, where
+// nothing else can modify the table meanwhile (else the call is noted with
+// the tracker for the kernels that follow); advances the arguments past the
+// keys it took, true if that is all. Tables whose inserts a process-wide
+// setting sends to another kernel family are left to it.
+template<class Core, class StatusHandler, bool HasValues, class Rec>
+WC_H bool insert_partitioned_first(const MutationTracker& mutations, const typename Core::key_type*& keys_in,
+                                   const typename Core::value_type*& values_in, index_t& num_in, const Core& core,
+                                   index_t probing_length, typename StatusHandler::base_type*& status_out,
+                                   hipStream_t stream, index_t table_bytes) noexcept {
+    if (!refill_inserts() || !owner_inserts() || table_bytes <= lane_insert_table_bytes() ||
+        !partition_pays<Core>(num_in, core.geometry())) {
+        mutations.note(stream);
+        return false;
+    }
+    MutationTracker::Exclusive exclusive(mutations, stream);
+    if (!exclusive.granted()) return false;
+    const index_t done = insert_partitioned<Core, StatusHandler, HasValues, Rec>(
+        keys_in, values_in, num_in, core, probing_length, status_out, stream);
+    if (done == 0) return false;
+    exclusive.use();
+    keys_in += done;
+    if constexpr (HasValues) values_in += done;
+    num_in -= done;
+    if constexpr (!std::is_same<StatusHandler, status_handlers::ReturnNothing>::value)
+        if (status_out != nullptr) status_out += done;
+    return num_in == 0;
 }
 
 }  // namespace detail

@@ -543,7 +543,10 @@ public:
         static_assert(checks::is_status_handler<StatusHandler>(), "not a valid status handler type");
         if (!is_initialized_ || num_in == 0) return;
         if constexpr (!soa_storage && detail::partition_capable<view_type>()) {
-            if (insert_partitioned<StatusHandler>(keys_in, values_in, num_in, stream, probing_length, status_out)) return;
+            if (detail::insert_partitioned_first<view_type, StatusHandler, true, slot_type>(
+                    mutations_, keys_in, values_in, num_in, state(), probing_length, status_out, stream,
+                    capacity() * sizeof(slot_type)))
+                return;
         } else {
             mutations_.note(stream);
         }
@@ -689,33 +692,6 @@ private:
         } else {
             return view_type{table_.data(), status_, geo_, seed_, is_initialized_, filter_valid_ ? filter_ : nullptr};
         }
-    }
-
-    // The partitioned insert of a batch that fills much of the table (see
-    // partition.hpp), where nothing else can modify the table meanwhile;
-    // advances the arguments past the keys it took, true if that is all.
-    template<class StatusHandler>
-    WC_H bool insert_partitioned(const key_type*& keys_in, const value_type*& values_in, index_type& num_in,
-                                 hipStream_t stream, index_type probing_length,
-                                 typename StatusHandler::base_type*& status_out) noexcept {
-        if (!detail::refill_inserts() || !detail::owner_inserts() ||
-            capacity() * sizeof(slot_type) <= detail::lane_insert_table_bytes() ||
-            !detail::partition_pays<view_type>(num_in, geo_)) {
-            mutations_.note(stream);
-            return false;
-        }
-        detail::MutationTracker::Exclusive exclusive(mutations_, stream);
-        if (!exclusive.granted()) return false;
-        const index_type done = detail::insert_partitioned<view_type, StatusHandler, true, slot_type>(
-            keys_in, values_in, num_in, state(), probing_length, status_out, stream);
-        if (done == 0) return false;
-        exclusive.use();
-        keys_in += done;
-        values_in += done;
-        num_in -= done;
-        if constexpr (!std::is_same<StatusHandler, status_handlers::ReturnNothing>::value)
-            if (status_out != nullptr) status_out += done;
-        return num_in == 0;
     }
 
     // Bulk kernels of AoS tables: lane-per-key windows on small tables,
