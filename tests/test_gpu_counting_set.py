@@ -246,3 +246,17 @@ def test_zipf_generator_distribution(cuda):
     pmf /= pmf.sum()
     exp = pmf[:8] * n
     assert np.all(np.abs(counts - exp) < 6 * np.sqrt(exp))
+
+
+def test_counting_erase_past_full_windows(cuda):
+    """At load 0.95 many keys sit past full windows; erase finds them all."""
+    from warpcore_amd.tables import CountingHashTable
+    n = 500_000
+    keys = unique_keys(n, 64, seed=31)
+    t = CountingHashTable(524_000, 64)
+    assert t.capacity() < 530_000
+    t.insert(to_dev(keys))
+    st = dev_empty(n, 32, 0x77)
+    t.erase(to_dev(keys), status_out=st)
+    assert (from_dev(st, np.uint32) == 0).all()
+    assert t.size() == 0

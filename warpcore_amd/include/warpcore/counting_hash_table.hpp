@@ -377,7 +377,12 @@ public:
     }
 
     // counting_hash_table.cuh:113-124; the EMPTY fill also zeroes the counters
-    WC_H void init(key_type seed, hipStream_t stream = 0) noexcept { base_table_.init(seed, stream); }
+    WC_H void init(key_type seed, hipStream_t stream = 0) noexcept {
+        base_table_.init(seed, stream);
+        // counting inserts do not keep the overflow filter, so the base
+        // table's erase must not end a walk by it
+        base_table_.filter_valid_ = false;
+    }
     WC_H void init(hipStream_t stream = 0) noexcept { init(base_table_.seed(), stream); }
 
     WC_D status_type insert(key_type key_in, const tile<cg_size()>& group,
