@@ -232,3 +232,20 @@ def test_counting_with_maximum(cuda):
     out = dev_empty(len(uniq), 64, 0)
     t.retrieve(to_dev(uniq), out)
     assert (from_dev(out, np.uint64) == 3).all()
+
+
+@pytest.mark.parametrize("kb,sb,num_bits,k,n,shape", [
+    (64, 64, 1 << 26, 8, 1 << 20, "distinct"),
+    (64, 64, (1 << 30) - 4096 * 64 + 64, 5, 3_000_017, "distinct"),   # 2048 regions, a short last one
+    (64, 32, 40_000_003, 4, 2_000_001, "hot"), (32, 64, 9_999_999, 7, 1_500_000, "few"),
+    (32, 32, (1 << 16) + 1, 3, (1 << 20) + 1, "distinct"),            # regions of one word
+])
+def test_bloom_insert(cuda, oracle, kb, sb, num_bits, k, n, shape):
+    from warpcore_amd.tables import BloomFilter
+    keys = _batch(n, kb, shape, seed=n)
+    bf = BloomFilter(num_bits, k, kb, slot_bits=sb)
+    ob = oracle.Bloom(num_bits, k, kb, sb, 1, bf.seed())
+    for part in (keys[: n // 2], keys):   # the second call on top of the first
+        bf.insert(to_dev(part))
+        ob.insert(part)
+        np.testing.assert_array_equal(from_dev(bf.words(), dtype(sb)), ob.words())

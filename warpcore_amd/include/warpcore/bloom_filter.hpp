@@ -24,6 +24,7 @@
 #include "engine.hpp"
 #include "fastmod.hpp"
 #include "hashers.hpp"
+#include "partition.hpp"
 #include "status.hpp"
 #include "tile.hpp"
 
@@ -32,6 +33,11 @@
 namespace warpcore {
 
 namespace detail {
+
+// Partitioned insert: keys per thread of a tile, most regions (whose LDS
+// bounds a region by kRegionBytes, the filter by 128 MB).
+constexpr unsigned kBloomItems = 8;
+constexpr unsigned kBloomRegions = 2048;
 
 template<class Key, class Hasher, class Slot, index_t CGSize>
 struct BloomView {
@@ -47,6 +53,9 @@ struct BloomView {
     index_t k;
     Key seed;
 
+    WC_D index_t block_of(Key key) const noexcept {
+        return mod_blocks.mod(std::uint64_t(Hasher::hash(Key(key + seed))));
+    }
     // word of `rank` in the key's block and the bits the key sets in it
     WC_D void locate(Key key, unsigned rank, index_t& slot_index, Slot& pattern) const noexcept {
         const Key seeded = Key(key + seed);
@@ -156,6 +165,96 @@ __global__ __launch_bounds__(256) void bloom_retrieve(const typename View::key_t
     }
 }
 
+// Partitioned insert (one word per key, CG = 1). The plain insert is bound by
+// its one memory-side OR per key (2^27 keys: 5.0 ms); here the keys are
+// sorted by region of the filter first (TileSort, partition.hpp), each region
+// is collected in LDS and ORed into the filter word by word, 206 G words/s
+// where the words follow each other. Scatter: a key without room in its
+// region's segment (many copies of one key) is ORed into the filter at once.
+template<class View>
+__global__ __launch_bounds__(1024, 4) void bloom_scatter(const typename View::key_type* __restrict__ keys_in,
+                                                         index_t num_in, View view, unsigned shift, unsigned regions,
+                                                         unsigned cap, typename View::key_type* __restrict__ out,
+                                                         std::uint32_t* __restrict__ counts) {
+    using K = typename View::key_type;
+    constexpr unsigned I = detail::kBloomItems;
+    __shared__ detail::TileSort<K, I, detail::kBloomRegions, false> ts;
+    const unsigned x = blockIdx.x % detail::kPartXcds;
+    constexpr index_t T = index_t(detail::kPartThreads) * I;
+    for (index_t tile = index_t(blockIdx.x) * T; tile < num_in; tile += index_t(gridDim.x) * T) {
+        ts.clear(regions);
+        K key[I];
+        std::uint32_t none[1], digit[I];
+#pragma unroll
+        for (unsigned j = 0; j < I; ++j) {
+            const index_t i = tile + j * detail::kPartThreads + threadIdx.x;
+            key[j] = i < num_in ? keys_in[i] : K{};
+        }
+#pragma unroll
+        for (unsigned j = 0; j < I; ++j) {
+            const index_t i = tile + j * detail::kPartThreads + threadIdx.x;
+            digit[j] = i < num_in ? std::uint32_t(view.block_of(key[j]) >> shift) : ~0u;
+        }
+        __syncthreads();
+        const index_t n = cap;
+        ts.append(
+            key, none, digit, regions, counts + x * regions, cap,
+            [=](std::uint32_t d) { return (index_t(d) * detail::kPartXcds + x) * n; }, out, nullptr,
+            [](std::uint32_t) { return index_t(0); },
+            [&](unsigned j, index_t) {
+                index_t at;
+                typename View::slot_type pattern;
+                view.locate(key[j], 0, at, pattern);
+                (void)__hip_atomic_fetch_or(view.words + at, pattern, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            });
+        __syncthreads();
+    }
+}
+
+// One region (1 << shift words) per block: its keys' patterns ORed in LDS,
+// then into the filter. Bound by hashing: k + 1 hashes per key (k = 8, 64-bit
+// keys: about 1 ms per 2^27 keys).
+template<class View>
+__global__ __launch_bounds__(1024, 8) void bloom_build(const typename View::key_type* __restrict__ in,
+                                                       const std::uint32_t* __restrict__ counts, View view,
+                                                       unsigned shift, unsigned regions, unsigned cap) {
+    using S = typename View::slot_type;
+    __shared__ S words[detail::kRegionBytes / sizeof(S)];
+    const unsigned per = 1u << shift;
+    for (unsigned r = blockIdx.x; r < regions; r += gridDim.x) {
+        for (unsigned i = threadIdx.x; i < per; i += detail::kPartThreads) words[i] = 0;
+        __syncthreads();
+        for (unsigned s = 0; s < detail::kPartXcds; ++s) {
+            const std::uint32_t have = counts[s * regions + r];
+            const std::uint32_t c = have < cap ? have : cap;
+            const auto* seg = in + (index_t(r) * detail::kPartXcds + s) * cap;
+            constexpr unsigned U = 4;   // keys per thread read ahead of the hashing
+            for (std::uint32_t lo = threadIdx.x; lo < c; lo += U * detail::kPartThreads) {
+                typename View::key_type key[U];
+#pragma unroll
+                for (unsigned u = 0; u < U; ++u) {
+                    const std::uint32_t i = lo + u * detail::kPartThreads;
+                    key[u] = seg[i < c ? i : lo];
+                }
+#pragma unroll
+                for (unsigned u = 0; u < U; ++u) {   // (past the end: the first key again, the same bits)
+                    index_t at;
+                    S pattern;
+                    view.locate(key[u], 0, at, pattern);
+                    (void)__hip_atomic_fetch_or(words + (at & (per - 1)), pattern, __ATOMIC_RELAXED,
+                                                __HIP_MEMORY_SCOPE_WORKGROUP);
+                }
+            }
+        }
+        __syncthreads();
+        for (unsigned i = threadIdx.x; i < per; i += detail::kPartThreads)
+            if (words[i] != 0)
+                (void)__hip_atomic_fetch_or(view.words + (index_t(r) << shift) + i, words[i], __ATOMIC_RELAXED,
+                                            __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+    }
+}
+
 // Bulk form of the device member insert_and_query (bloom_filter.cuh:263-297):
 // one lane per key (CG = 1); flag = all of the key's bits were set before
 // its own atomicOr.
@@ -198,6 +297,7 @@ public:
           mod_slots_(num_slots_ ? num_slots_ : 1), k_(k), seed_(seed), is_copy_(false) {
         if (num_slots_ != 0 && hipMalloc(&bloom_filter_, sizeof(slot_type) * num_slots_) != hipSuccess)
             bloom_filter_ = nullptr;
+        detail::WorkspacePool::instance().add_user();
         init();
     }
     WC_HD BloomFilter(const BloomFilter& o) noexcept
@@ -213,6 +313,7 @@ public:
     WC_HD ~BloomFilter() noexcept {
 #if !defined(__HIP_DEVICE_COMPILE__)
         if (!is_copy_ && bloom_filter_ != nullptr) (void)hipFree(bloom_filter_);
+        if (!is_copy_) detail::WorkspacePool::instance().remove_user();
 #endif
     }
 
@@ -235,6 +336,8 @@ public:
     // bloom_filter.cuh:199-208
     WC_H void insert(const key_type* keys_in, index_type num_in, hipStream_t stream = 0) noexcept {
         if (bloom_filter_ == nullptr || num_in == 0) return;
+        if constexpr (CGSize == 1)
+            if (insert_partitioned(keys_in, num_in, stream)) return;
         kernels::bloom_insert<view_type, 4>
             <<<detail::grid_for(SDIV(num_in, 4), cg_size()), block_size(), 0, stream>>>(keys_in, num_in, view());
     }
@@ -281,6 +384,56 @@ public:
     }
 
 private:
+    // The insert of a batch large enough to sort: at least 2^20 keys (the
+    // plain insert takes 40 us for as many, the two sorted passes and their
+    // launches as long), and a sixteenth of the words (every word is ORed
+    // once). Filters up to 128 MB. Under capture the workspace, which is only
+    // leased, could not be kept for the graph's replays.
+    WC_H bool insert_partitioned(const key_type* keys_in, index_type num_in, hipStream_t stream) noexcept {
+        constexpr unsigned largest = unsigned(detail::kRegionBytes / sizeof(slot_type));
+        if (num_in < (index_type(1) << 20) || num_in < num_slots_ / 16 ||
+            num_slots_ > index_type(largest) * detail::kBloomRegions)
+            return false;
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(stream, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) {
+            (void)hipGetLastError();
+            return false;
+        }
+        unsigned shift = 0;   // up to 1024 regions, or 2048 of the largest
+        while ((num_slots_ >> shift) >= detail::kBloomRegions / 2 && (1u << shift) < largest) ++shift;
+        const unsigned regions = unsigned(SDIV(num_slots_, index_type(1) << shift));
+        constexpr index_type tile = index_type(detail::kPartThreads) * detail::kBloomItems;
+        for (index_type done = 0; done < num_in;) {
+            const index_type n = std::min(num_in - done, detail::kPartChunk);
+            const index_type tiles = SDIV(n, tile);
+            const double share = std::min(double(SDIV(tiles, index_type(detail::kPartXcds)) * tile), double(n));
+            const unsigned cap = detail::part_capacity(share * std::min(1.0, double(index_type(1) << shift) /
+                                                                                 double(num_slots_)));
+            const index_type count_bytes = index_type(regions) * detail::kPartXcds * 4;
+            detail::WorkspaceLease ws(count_bytes + index_type(regions) * detail::kPartXcds * cap * sizeof(key_type),
+                                      stream);
+            if (!ws) {
+                if (done == 0) return false;
+                kernels::bloom_insert<view_type, 4>
+                    <<<detail::grid_for(SDIV(num_in - done, 4), cg_size()), block_size(), 0, stream>>>(
+                        keys_in + done, num_in - done, view());
+                return true;
+            }
+            auto* counts = static_cast<std::uint32_t*>(ws.get());
+            auto* keys = reinterpret_cast<key_type*>(static_cast<unsigned char*>(ws.get()) + count_bytes);
+            storage::kernels::fill<std::uint32_t><<<detail::grid_for(count_bytes / 4, 1, 8), block_size(), 0, stream>>>(
+                counts, count_bytes / 4, 0u);
+            constexpr auto scatter = kernels::bloom_scatter<view_type>;
+            scatter<<<detail::part_grid<scatter>(tiles), detail::kPartThreads, 0, stream>>>(
+                keys_in + done, n, view(), shift, regions, cap, keys, counts);
+            constexpr auto build = kernels::bloom_build<view_type>;
+            build<<<detail::part_grid<build>(regions), detail::kPartThreads, 0, stream>>>(keys, counts, view(), shift,
+                                                                                          regions, cap);
+            done += n;
+        }
+        return true;
+    }
+
     slot_type* bloom_filter_;
     index_type num_bits_;
     index_type num_slots_;
