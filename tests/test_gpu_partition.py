@@ -222,6 +222,28 @@ def test_counting_insert(cuda, kb, n, distinct, skew, statuses):
     np.testing.assert_array_equal(from_dev(found, np.uint32) == S_NONE, total > 0)
 
 
+@pytest.mark.parametrize("kb", [32, 64])
+@pytest.mark.parametrize("n", [(1 << 22) - 1, 1 << 22, (1 << 23) + 8191])
+@pytest.mark.parametrize("shape", ["one", "few", "distinct"])
+def test_counting_large_pass(cuda, kb, n, shape):
+    """Combining without statuses at the size where a pass takes the larger
+    tile: one key only, a few, as many as occurrences; invalid keys between."""
+    from warpcore_amd.tables import CountingHashTable
+    distinct = {"one": 1, "few": 3000, "distinct": n}[shape]
+    uniq = unique_keys(distinct, kb, seed=n + 1)
+    pick = np.random.default_rng(n).permutation(n) % distinct
+    keys = uniq[pick]
+    bad = np.array([5, n // 2, n - 1])
+    keys[bad] = [0, np.iinfo(keys.dtype).max, 0]
+    t = CountingHashTable(math.ceil(distinct / 0.9) + 64, kb)
+    t.insert(to_dev(keys))
+    total = np.bincount(np.delete(pick, bad), minlength=distinct)
+    out = dev_empty(distinct, 64, 0)
+    t.retrieve(to_dev(uniq), out)
+    np.testing.assert_array_equal(from_dev(out, np.int64) * (total > 0), total)
+    assert t.size() == (total > 0).sum()
+
+
 def test_counting_with_maximum(cuda):
     """A maximum count: the general insert, which stops there."""
     from warpcore_amd.tables import CountingHashTable
