@@ -14,6 +14,7 @@ from datagen import dev_empty, dtype, from_dev, to_dev, tomb, uniform_values, un
 pytestmark = pytest.mark.gpu
 
 S_NONE, S_PLE, S_INVALID_KEY, S_DUP, S_NOT_FOUND = 0, 2, 8, 16, 32
+S_OUT_OF_MEMORY, S_MAX_VALUES = 1 << 7, 1 << 11
 SENTINEL = 0x5A5A5A5A
 
 
@@ -271,3 +272,102 @@ def test_bloom_insert(cuda, oracle, kb, sb, num_bits, k, n, shape):
         bf.insert(to_dev(part))
         ob.insert(part)
         np.testing.assert_array_equal(from_dev(bf.words(), dtype(sb)), ob.words())
+
+
+def _pair_batch(n, bits, distinct, shape, seed):
+    """n pairs over `distinct` keys with distinct values, some keys invalid."""
+    rng = np.random.default_rng(seed)
+    uniq = unique_keys(distinct, bits, seed=seed + 1)
+    if shape == "heavy":     # a share of the batch on few keys: the general insert takes it
+        w = np.arange(1, distinct + 1, dtype=np.float64) ** -1.2
+        pick = np.searchsorted(np.cumsum(w / w.sum()), rng.random(n)).clip(max=distinct - 1)
+    else:
+        pick = rng.integers(0, distinct, n)
+        if shape == "warm":  # a few keys of some thousand pairs, too few to be sampled
+            pick[: n // 16] = rng.integers(0, max(1, n // 16 // 3000), n // 16)
+    keys = uniq[pick]
+    if shape == "invalid":
+        keys[::9973] = 0
+        keys[1::9967] = tomb(bits)
+    return np.ascontiguousarray(keys), np.arange(1, n + 1).astype(dtype(bits)), uniq
+
+
+def _values_by_key(t, uniq, bits, total):
+    """Every key's values, sorted, from one retrieve."""
+    begin, end = dev_empty(len(uniq), 64, 0), dev_empty(len(uniq), 64, 0)
+    out = dev_empty(total + 1, bits, 0)
+    assert t.retrieve(to_dev(uniq), begin, end, out[:total]) == total
+    b, e, v = from_dev(begin, np.int64), from_dev(end, np.int64), from_dev(out, dtype(bits))[:total]
+    assert b[0] == 0 and e[-1] == total and (b[1:] == e[:-1]).all()
+    owner = np.repeat(np.arange(len(uniq)), e - b)
+    return owner, v[np.lexsort((v, owner))]
+
+
+def _expected_by_key(keys, values, uniq):
+    order = np.argsort(uniq, kind="stable")
+    at = np.searchsorted(uniq[order], keys)
+    pos = order[at.clip(max=len(uniq) - 1)]
+    ok = uniq[pos] == keys
+    owner, v = pos[ok], values[ok]
+    by = np.lexsort((v, owner))
+    return owner[by], v[by]
+
+
+@pytest.mark.parametrize("bits,n,distinct,shape", [
+    (32, 1 << 20, 1 << 17, "even"), (32, (1 << 20) + 1, 1 << 20, "invalid"), (32, 3_000_017, 300_000, "warm"),
+    (32, 1_500_000, 50_000, "heavy"), (64, (1 << 20) + 4097, 90_001, "invalid"), (64, (1 << 23) + 5, 3_000_000, "even"),
+])
+def test_pairs_insert(cuda, bits, n, distinct, shape):
+    """Two calls, the second on top of the first's keys."""
+    from warpcore_amd.tables import BucketListHashTable
+    keys, values, uniq = _pair_batch(n, bits, distinct, shape, seed=n)
+    t = BucketListHashTable(math.ceil(distinct / 0.9) + 64, 4 * n + 4096, bits, bits)
+    ok = _valid(keys, bits)
+    stored = len(np.unique(keys[ok]))
+    for call in range(2):
+        t.insert(to_dev(keys), to_dev(values))
+        status = int(t.pop_status())
+        assert status & ~(S_DUP | S_INVALID_KEY) == 0
+        assert bool(status & S_INVALID_KEY) == (not ok.all())
+        assert t.num_keys() == stored
+        want = _expected_by_key(np.tile(keys[ok], call + 1), np.tile(values[ok], call + 1), uniq)
+        got = _values_by_key(t, uniq, bits, (call + 1) * int(ok.sum()))
+        t.pop_status()   # key_not_found of the keys that the batch does not hold
+        np.testing.assert_array_equal(got[0], want[0])
+        np.testing.assert_array_equal(got[1], want[1])
+
+
+@pytest.mark.parametrize("min_size,grow,max_size", [(1, 1.0, 1), (3, 1.1, 1023), (8, 2.0, 64), (1, 1.001, 1023)])
+def test_pairs_insert_bucket_shapes(cuda, min_size, grow, max_size):
+    from warpcore_amd.tables import BucketListHashTable
+    n, distinct = 1_300_000, 60_000
+    keys, values, uniq = _pair_batch(n, 32, distinct, "even", seed=7)
+    t = BucketListHashTable(70_000, 6 * n, 32, 32, grow_factor=grow, min_bucket_size=min_size, max_bucket_size=max_size)
+    for call in range(2):
+        t.insert(to_dev(keys), to_dev(values))
+    assert int(t.pop_status()) == S_DUP
+    want = _expected_by_key(np.tile(keys, 2), np.tile(values, 2), uniq)
+    got = _values_by_key(t, uniq, 32, 2 * n)
+    np.testing.assert_array_equal(got[0], want[0])
+    np.testing.assert_array_equal(got[1], want[1])
+
+
+def test_pairs_insert_limits(cuda):
+    """A per-key maximum, and a pool too small for the batch."""
+    from warpcore_amd.tables import BucketListHashTable
+    n, distinct = 1_200_000, 60_000
+    keys, values, uniq = _pair_batch(n, 32, distinct, "even", seed=9)
+    have = np.bincount(np.searchsorted(np.sort(uniq), keys), minlength=distinct)
+    t = BucketListHashTable(70_000, 4 * n, 32, 32, max_values_per_key=10)
+    t.insert(to_dev(keys), to_dev(values))
+    assert int(t.pop_status()) == S_DUP | S_MAX_VALUES
+    owner, v = _values_by_key(t, np.sort(uniq), 32, int(np.minimum(have, 10).sum()))
+    np.testing.assert_array_equal(np.bincount(owner, minlength=distinct), np.minimum(have, 10))
+    assert len(np.unique(v)) == len(v) and (np.sort(uniq)[owner] == keys[v.astype(np.int64) - 1]).all()
+    small = BucketListHashTable(70_000, n // 2, 32, 32)
+    small.insert(to_dev(keys), to_dev(values))
+    assert int(small.pop_status()) & (S_OUT_OF_MEMORY | S_DUP) == S_OUT_OF_MEMORY | S_DUP
+    total = small.num_values()
+    assert n // 8 < total <= n // 2
+    owner, v = _values_by_key(small, uniq, 32, total)
+    assert len(np.unique(v)) == total and (uniq[owner] == keys[v.astype(np.int64) - 1]).all()

@@ -37,6 +37,7 @@
 #include "defaults.hpp"
 #include "engine.hpp"
 #include "multi_value_hash_table.hpp"
+#include "pair_groups.hpp"
 #include "scan.hpp"
 #include "single_value_hash_table.hpp"
 #include "status.hpp"
@@ -151,12 +152,15 @@ struct BucketListStoreView {
         return a + 1 < arenas ? arena_cells : capacity - a * arena_cells;
     }
 
+    WC_D index_t home_arena() const noexcept {
+        return arenas == 1 ? 0 : index_t(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) & (arenas - 1);
+    }
+
     // `n` cells for every active lane, from the wavefront's home arena or
     // the ones after it; the first cell, or ~0 when no arena holds them.
     // Active lanes take part together (a wave-uniform walk over the arenas).
     WC_D index_t allocate(index_t n) const noexcept {
-        const index_t home = arenas == 1 ? 0
-            : index_t(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) & (arenas - 1);
+        const index_t home = home_arena();
         for (index_t t = 0; t < arenas; ++t) {
             const index_t a = (home + t) & (arenas - 1);
             const index_t at = wave_atomic_add(counters + a * kCounterStride, n);
@@ -189,18 +193,25 @@ struct BucketListStoreView {
     // does), so it is found from the count without reading the bucket's link
     // when the sequence settles within kSizeSteps steps; false otherwise.
     static constexpr int kSizeSteps = 64;
-    WC_D bool size_by_count(index_t c, index_t& size) const noexcept {
-        index_t cum = min_size;
-        size = min_size;
+    // counts and sizes of one key: 32 bits where the handle's fields allow
+    // (the sequence is computed per append and per bucket walked)
+    using small_type = typename std::conditional<(CB < 32 && SB < 32), std::uint32_t, index_t>::type;
+    WC_D bool size_by_count(index_t count, index_t& size_out) const noexcept {
+        const small_type c = small_type(count);
+        small_type size = small_type(min_size), cum = size;
         for (int k = 0; k < kSizeSteps && cum < c; ++k) {
-            const index_t next = grown(size);
-            if (next == size) return true;   // the same size from here on
+            const small_type next = grown(size);
+            if (next == size) break;   // the same size from here on
             size = next;
             cum += size;
+            if (k + 1 == kSizeSteps && cum < c) return false;
         }
-        return cum >= c;
+        size_out = size;
+        return true;
     }
-    WC_D index_t grown(index_t size) const noexcept { return index_t(fminf(float(max_size), ceilf(float(size) * grow))); }
+    WC_D small_type grown(small_type size) const noexcept {
+        return small_type(fminf(float(max_size), ceilf(float(size) * grow)));
+    }
 
     WC_D Status append(handle_type* handle, const Value& value, index_t max_values_per_key) const noexcept {
         return append_from(handle, warpcore::detail::atomic_load_relaxed(&handle->pack), value, max_values_per_key);
@@ -273,6 +284,173 @@ struct BucketListStoreView {
             }
         }
         return Status::unknown_error();
+    }
+
+    // State of a handle that the calling lane holds blocked.
+    struct Held {
+        index_t bucket;
+        small_type count, tail, size;   // size of the tail bucket, min_size while there is none
+    };
+    WC_D Held held(const handle_type& cur) const noexcept {
+        Held h{head(), 0, 0, small_type(min_size)};
+        if (cur.is_uninitialized()) return h;
+        h.bucket = cur.bucket_index();
+        h.count = small_type(cur.value_count());
+        h.tail = small_type(cur.num_values_tail());
+        index_t size = min_size;
+        if (h.count > min_size && !size_by_count(h.count, size))
+            size = bucket_type::size_of(warpcore::detail::atomic_load_relaxed(&buckets[h.bucket].info));
+        h.size = small_type(size);
+        return h;
+    }
+    WC_D static handle_type blocked(const handle_type& cur) noexcept {
+        if (cur.is_uninitialized()) return handle_type::make(detail::LinkedListState::blocking, head(), 0, 0);
+        return handle_type::make(detail::LinkedListState::blocking, cur.bucket_index(), cur.value_count(),
+                                 cur.num_values_tail());
+    }
+
+    // The values next(value) gives (until it returns false; `pairs` of them)
+    // appended to a held handle, buckets allocated and filled as append_from
+    // does value by value, first from the `cells` cells from `run` on;
+    // publishes the handle.
+    template<class Next>
+    WC_D Status fill(std::uint64_t* hp, Held h, const Next& next, small_type pairs, index_t max_values_per_key,
+                     index_t run, std::uint32_t cells) const noexcept {
+        using LS = detail::LinkedListState;
+        Status st = Status::none();
+        LS state = LS::initialized;
+        const small_type most = small_type(max_values_per_key);
+        const small_type first = small_type(min_size);
+        index_t known = 0;
+        const bool sized = size_by_count(index_t(h.count) + pairs, known);   // then every count before it is
+        bucket_type* to = buckets + h.bucket + (h.count > first ? 1 : 0) + h.tail;   // the next value's cell
+        small_type room = h.count == 0 ? 0 : h.size - h.tail;
+        Value value{};
+        while (next(value)) {
+            if (h.count == most) {
+                st = Status::max_values_for_key_reached();
+                break;
+            }
+            if (room == 0) {
+                const bool headed = h.count != 0;
+                const small_type larger = headed ? grown(h.size) : first;
+                const std::uint32_t need = std::uint32_t(larger) + (headed ? 1 : 0);
+                index_t alloc = run;
+                if (need <= cells) {
+                    run += need;
+                    cells -= need;
+                } else {
+                    alloc = allocate(index_t(larger) + (headed ? 1 : 0));
+                }
+                if (alloc == ~index_t(0)) {
+                    st = Status::out_of_memory();
+                    state = LS::full;
+                    break;
+                }
+                to = buckets + alloc;
+                if (headed) {
+                    const std::uint64_t link = bucket_type::make_info(h.bucket, larger);
+                    if (sized) to->info = link;   // read only by later launches: a plain store
+                    else wait_for(warpcore::detail::atomic_exch(&to->info, link));   // appends will read this link
+                    ++to;
+                }
+                h.bucket = alloc;
+                h.size = room = larger;
+            }
+            to->value = value;
+            ++to;
+            --room;
+            ++h.count;
+        }
+        const small_type tail = h.count == 0 ? 0 : h.size - room;
+        warpcore::detail::atomic_exch(hp, handle_type::make(state, h.bucket, h.count, tail).pack);
+        return st;
+    }
+
+    // Appends of several values to one handle, which is blocked once; returns
+    // the flags that appends one by one would have joined. No lane waits for
+    // another while it holds a handle: a blocked handle is always released.
+    template<class Next>
+    WC_D Status append_all(handle_type* handle, const Next& next, small_type pairs,
+                           index_t max_values_per_key) const noexcept {
+        std::uint64_t* hp = &handle->pack;
+        std::uint64_t seen = warpcore::detail::atomic_load_relaxed(hp);
+        for (std::uint32_t reads = 0; reads < kMaxBlockedReads; ++reads) {
+            const handle_type cur{seen};
+            if (cur.is_blocking()) {   // another lane is appending: wait a little
+                __builtin_amdgcn_s_sleep(1);
+                seen = warpcore::detail::atomic_load_relaxed(hp);
+                continue;
+            }
+            if ((cur.is_uninitialized() ? 0 : cur.value_count()) >= max_values_per_key)
+                return Status::max_values_for_key_reached();
+            if (cur.is_full()) return Status::out_of_memory();
+            seen = warpcore::detail::atomic_cas(hp, cur.pack, blocked(cur).pack);
+            if (seen == cur.pack) return fill(hp, held(cur), next, pairs, max_values_per_key, 0, 0);
+        }
+        return Status::unknown_error();
+    }
+
+    // append_all of `pairs` values for every lane with `on`; all lanes of the
+    // wavefront call this. The lanes that block their handle at the first
+    // try have the cells of all their buckets allocated by one atomic, where
+    // the wavefront's arena holds them (2^26 pairs over 2^23 keys: the groups
+    // pass 3.65 ms, bucket by bucket, an atomic's round trip each, 4.07); the
+    // others append on their own after those have published.
+    // (`fresh`: the handle of a key just claimed, taken to be uninitialised.)
+    template<class Next>
+    WC_D Status append_wave(bool on, bool fresh, handle_type* handle, small_type pairs, const Next& next,
+                            index_t max_values_per_key) const noexcept {
+        Status st = Status::none();
+        bool mine = false;
+        Held h{head(), 0, 0, small_type(min_size)};
+        if (on) {
+            handle_type cur = handle_type::make(detail::LinkedListState::uninitialized, head(), 0, 0);
+            if (!fresh) cur = handle_type{warpcore::detail::atomic_load_relaxed(&handle->pack)};
+            if (!cur.is_blocking() && !cur.is_full() &&
+                (cur.is_uninitialized() ? 0 : cur.value_count()) < max_values_per_key) {
+                mine = warpcore::detail::atomic_cas(&handle->pack, cur.pack, blocked(cur).pack) == cur.pack;
+                if (mine) h = held(cur);
+            }
+        }
+        std::uint32_t cells = 0;
+        if (mine) {
+            bool headed = h.count != 0;
+            small_type size = h.size, room = headed ? size - h.tail : 0;
+            const small_type most = small_type(max_values_per_key) - h.count;
+            small_type more = most < pairs ? most : pairs;
+            while (more > room && cells < (1u << 20)) {
+                more -= room;
+                room = size = headed ? grown(size) : small_type(min_size);
+                cells += std::uint32_t(size) + (headed ? 1 : 0);
+                headed = true;
+            }
+        }
+        std::uint32_t upto = cells;
+#pragma unroll
+        for (unsigned s = 1; s < 64; s <<= 1) {
+            const std::uint32_t o = __shfl_up(upto, s, 64);
+            if (warpcore::lane_id() >= s) upto += o;
+        }
+        const std::uint32_t total = unsigned(__builtin_amdgcn_readlane(int(upto), 63));
+        index_t run = ~index_t(0);
+        if (total != 0) {   // uniform
+            const index_t a = home_arena();
+            if (warpcore::lane_id() == 0) {
+                index_t* counter = counters + a * kCounterStride;
+                if (warpcore::detail::atomic_load_relaxed(counter) + total <= arena_size(a)) {
+                    const index_t at = warpcore::detail::atomic_add(counter, index_t(total));
+                    if (at + total <= arena_size(a)) run = arena_begin(a) + at;
+                }
+            }
+            run = (index_t(unsigned(__builtin_amdgcn_readfirstlane(int(run >> 32)))) << 32) |
+                  index_t(unsigned(__builtin_amdgcn_readfirstlane(int(run))));
+        }
+        if (mine)
+            st = fill(&handle->pack, h, next, pairs, max_values_per_key, run + (upto - cells),
+                      run != ~index_t(0) ? cells : 0u);
+        if (on && !mine) st = append_all(handle, next, pairs, max_values_per_key);
+        return st;
     }
 
     // f(value, j) for j < count, lanes of `group` striding over the values
@@ -601,9 +779,210 @@ struct BucketListKeyCore : KeyView {
     }
 };
 
+// Key walk of up to 64 keys of a wavefront: the slot of key `first` + i goes
+// to out[i] (it keeps its value where the key failed).
+template<class KeyView>
+struct BucketListSlotCore : KeyView {
+    std::uint32_t* out;
+    index_t first;
+    template<class Join>
+    WC_D void finish_insert(index_t, const typename KeyView::value_type&, bool, Status&, Join&) const noexcept {}
+    WC_D void on_slot(index_t slot, index_t pos, bool) const noexcept { out[pos - first] = std::uint32_t(slot); }
+};
+
+// Insert of grouped pairs (pair_groups.hpp): a wavefront finds or claims the
+// slots of up to 64 keys, then each lane appends all pairs of its key.
+// Pair by pair an append costs one memory-side compare-and-swap on the
+// handle and another round trip where a bucket is linked; per key of the
+// region it is two. The first step of every key's walk reads the region's keys
+// in LDS (2.6 ms for the groups pass, with the walks in the table 3.1). 2^26
+// pairs over 2^23 keys: key pass 2.1 and appends 4.8 ms pair by pair; sorted
+// and grouped 3.4 ms.
+template<class KeyView, class StoreView>
+struct BucketListGroupCore : KeyView {
+    using key_type = typename KeyView::key_type;
+    using pair_value_type = typename StoreView::value_type;
+    static constexpr unsigned most_region_slots = 1024;
+    StoreView store;
+    index_t max_values;
+
+    template<unsigned N>
+    struct WalkScratch {
+        OwnerEntry<key_type, std::uint32_t> entry[N];
+        std::uint32_t slot[N];
+    };
+    struct group_scratch : WalkScratch<kPartThreads> {
+        alignas(16) key_type key[most_region_slots];   // keys of the region's slots
+        std::uint16_t moved[kPartThreads];       // per wavefront: its keys that go on to their second window
+    };
+    using rest_scratch = WalkScratch<256>;
+
+    WC_D index_t budget(index_t probing_length) const noexcept {
+        return probing_schemes::detail::window_budget(probing_length, KeyView::cg_size(), this->geometry().windows);
+    }
+
+    // slots of keys [first, end) of `in`, at most 64, into the wavefront's
+    // scratch.slot (~0 for a key that failed)
+    template<class Input, unsigned N, class Join>
+    WC_D void find_slots(const Input& in, index_t first, index_t end, WalkScratch<N>& scratch, index_t windows,
+                         Join& join) const noexcept {
+        const unsigned wave = threadIdx.x & ~63u;
+        scratch.slot[threadIdx.x] = ~0u;
+        wave_sync();
+        const BucketListSlotCore<KeyView> core{*this, scratch.slot + wave, first};
+        insert_owner_from<BucketListSlotCore<KeyView>, status_handlers::ReturnNothing, std::uint32_t, false,
+                          part_spl<BucketListSlotCore<KeyView>>()>(in, first, end, core, windows, nullptr,
+                                                                   scratch.entry + wave, join);
+        wave_sync();
+    }
+    WC_D static void wave_sync() noexcept {   // LDS written by the wavefront's other lanes
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+
+    // Keys of a round that a wavefront moves on to their second windows.
+    template<class Rec>
+    struct MovedInput {
+        const PairGroups<Rec>* groups;
+        const std::uint16_t* list;
+        static constexpr bool skip_first = true;
+        WC_D key_type key(index_t i) const noexcept { return groups->key(list[i]); }
+        WC_D typename KeyView::value_type value(index_t) const noexcept { return {}; }
+        WC_D static index_t position(index_t i) noexcept { return i; }
+    };
+
+    // The keys of the region's slots, before its first round: every key's
+    // first window lies here, so the walks' first steps read LDS.
+    WC_D void begin_region(group_scratch& scratch, index_t w0, unsigned region_windows) const noexcept {
+        constexpr unsigned CG = unsigned(KeyView::cg_size());
+        const index_t windows = this->geometry().windows;
+        const unsigned slots = unsigned(windows - w0 < region_windows ? windows - w0 : region_windows) * CG;
+        for (unsigned i = threadIdx.x; i < slots; i += kPartThreads)
+            scratch.key[i] = this->slots[w0 * CG + i].key;
+    }
+
+    // The lane's key in its first window: the slot, `claimed` if it is new
+    // there, or ~0 when the window is full. Claims settle in LDS first, so
+    // that one lane asks the table for a slot; a slot that a key of another
+    // region took meanwhile, on its way past its own first window, is
+    // corrected here and passed by. (A key passes slots that others are still
+    // claiming: no call beside this one may insert, or it could put the same
+    // key there.)
+    WC_D std::uint32_t first_step(key_type key, group_scratch& scratch, index_t w, index_t w0,
+                                  bool& claimed) const noexcept {
+        constexpr unsigned CG = unsigned(KeyView::cg_size());
+        const unsigned at = unsigned(w - w0) * CG;
+        unsigned hit = CG, empty = CG;
+#pragma unroll
+        for (unsigned o = CG; o-- > 0;) {
+            const key_type k = scratch.key[at + o];
+            if (k == key) hit = o;
+            if (KeyView::is_empty_key(k)) empty = o;
+        }
+        const index_t slot = w * CG;
+        if (hit < CG) return std::uint32_t(slot + hit);
+        for (unsigned o = empty; o < CG; ++o) {
+            const key_type there = scratch.key[at + o];
+            if (!KeyView::is_empty_key(there) || !KeyView::is_empty_key(atomic_cas(scratch.key + at + o, there, key)))
+                continue;
+            const key_type old = atomic_cas(&this->slots[slot + o].key, there, key);
+            claimed = old == there;
+            if (claimed || old == key) return std::uint32_t(slot + o);
+            scratch.key[at + o] = old;
+        }
+        return ~0u;
+    }
+
+    template<class Rec, class Join>
+    WC_D void insert_groups(const PairGroups<Rec>& groups, group_scratch& scratch, index_t w0,
+                            index_t probing_length, Join& join) const noexcept {
+        const std::uint32_t num = groups.groups;
+        constexpr std::uint32_t waves = kPartThreads / 64;
+        const unsigned wave = threadIdx.x & ~63u;
+        const std::uint32_t share = (num + waves - 1) / waves;   // few keys: fewer per wavefront, all at work
+        const std::uint32_t per = share < 64 ? share : 64;
+        const index_t windows = budget(probing_length);
+        for (std::uint32_t g0 = threadIdx.x / 64 * per; g0 < num; g0 += waves * per) {
+            const std::uint32_t g = g0 + lane_id();
+            bool on = g < (g0 + per < num ? g0 + per : num) && this->ready();
+            bool claimed = false;
+            unsigned at = 0, end = 0, pairs = 0;
+            key_type key{};
+            std::uint32_t slot = ~0u;
+            if (on) {
+                key = groups.key(g);
+                at = groups.list[g];
+                end = groups.end(g);
+                WindowCursor<typename KeyView::probing_scheme_type> c;
+                c.begin(key, this->hash_seed(), this->geometry());
+                slot = first_step(key, scratch, c.w, w0, claimed);
+                if (slot == ~0u) mark_overflow(static_cast<const KeyView&>(*this), std::uint32_t(c.w), std::uint32_t(c.step));
+                if (!claimed && slot != ~0u) join(Status::duplicate_key());
+                for (unsigned q = at; q < end; ++q) pairs += groups.buf[q].key == key;
+                if (pairs > 1) join(Status::duplicate_key());   // all but one found the key
+            }
+            const std::uint64_t go = __builtin_amdgcn_ballot_w64(on && slot == ~0u);
+            if (go != 0) {
+                const unsigned mine = lanes_below(go);
+                if (on && slot == ~0u) scratch.moved[wave + mine] = std::uint16_t(g);
+                wave_sync();
+                const MovedInput<Rec> in{&groups, scratch.moved + wave};
+                find_slots(in, 0, index_t(__builtin_popcountll(go)), scratch, windows, join);
+                if (on && slot == ~0u) slot = scratch.slot[wave + mine];
+                wave_sync();
+            }
+            on = on && slot != ~0u;
+            const Status st = store.append_wave(
+                on, claimed, &this->slots[on ? slot : 0].value, pairs,
+                [&](pair_value_type& v) {
+                    while (at < end && groups.buf[at].key != key) ++at;
+                    if (at >= end) return false;
+                    v = groups.buf[at++].value;
+                    return true;
+                },
+                max_values);
+            if (st.has_any()) join(st);
+        }
+    }
+
+    template<class Input, class Join>
+    WC_D void insert_pairs(const Input& in, index_t lo, index_t hi, rest_scratch& scratch, index_t probing_length,
+                           Join& join) const noexcept {
+        const index_t windows = budget(probing_length);
+        for (index_t i0 = lo; i0 < hi; i0 += 64) {
+            const index_t i1 = i0 + 64 < hi ? i0 + 64 : hi;
+            find_slots(in, i0, i1, scratch, windows, join);
+            const std::uint32_t slot = scratch.slot[threadIdx.x];
+            wave_sync();
+            const index_t i = i0 + lane_id();
+            if (i >= i1 || slot == ~0u) continue;
+            bool more = true;
+            const Status st = store.append_all(
+                &this->slots[slot].value,
+                [&](pair_value_type& v) {
+                    if (!more) return false;
+                    v = in.value(i);
+                    more = false;
+                    return true;
+                },
+                1, max_values);
+            if (st.has_any()) join(st);
+        }
+    }
+};
+
 }  // namespace detail
 
 namespace kernels {
+
+// slot_of of a chunk before its key pass: no slot
+__global__ __launch_bounds__(256) inline void bl_clear(std::uint32_t* __restrict__ slot_of, index_t num_in,
+                                                       const index_t* __restrict__ num_dev) {
+    if (num_dev != nullptr && *num_dev < num_in) num_in = *num_dev;
+    const index_t stride = index_t(gridDim.x) * blockDim.x;
+    for (index_t i = index_t(blockIdx.x) * blockDim.x + threadIdx.x; i < num_in; i += stride) slot_of[i] = ~0u;
+}
 
 // Append pass of a bucket-list insert: one lane per pair, the pair's value
 // appended to the handle of the slot the key pass recorded (the appends of
@@ -614,9 +993,11 @@ template<class View, class StatusHandler>
 __global__ __launch_bounds__(256) void bl_append(const typename View::value_type* __restrict__ values_in,
                                                  index_t num_in, const std::uint32_t* __restrict__ slot_of,
                                                  const Status* __restrict__ key_status, View view,
-                                                 typename StatusHandler::base_type* __restrict__ status_out) {
+                                                 typename StatusHandler::base_type* __restrict__ status_out,
+                                                 const index_t* __restrict__ num_dev) {
     using handle_type = typename View::handle_type;
     warpcore::detail::DeferredJoin join;
+    if (num_dev != nullptr && *num_dev < num_in) num_in = *num_dev;
     const index_t stride = index_t(gridDim.x) * blockDim.x;
     for (index_t i = index_t(blockIdx.x) * blockDim.x + threadIdx.x; i < num_in; i += stride) {
         const std::uint32_t slot = slot_of[i];
@@ -837,14 +1218,14 @@ public:
     WC_D status_type insert(key_type key_in, const value_type& value_in, const tile<cg_size()>& group,
                             index_type probing_length = defaults::probing_length()) const noexcept {
         warpcore::detail::ImmediateJoin join{hash_table_.status_};
-        return view().insert(key_in, value_in, group, probing_length, join);
+        return state().insert(key_in, value_in, group, probing_length, join);
     }
     WC_D status_type retrieve(key_type key_in, value_type* values_out, index_type& num_out,
                               const tile<cg_size()>& group,
                               index_type probing_length = defaults::probing_length()) const noexcept {
         warpcore::detail::ImmediateJoin join{hash_table_.status_};
         handle_type h{0};
-        const status_type st = view().find(key_in, h, group, probing_length, join);
+        const status_type st = state().find(key_in, h, group, probing_length, join);
         if (!st.has_any()) {
             value_store_.for_each([=](const value_type& v, index_type j) { values_out[j] = v; }, h, group);
             num_out = h.value_count();
@@ -858,7 +1239,7 @@ public:
                               index_type probing_length = defaults::probing_length()) const noexcept {
         warpcore::detail::ImmediateJoin join{hash_table_.status_};
         handle_type h{0};
-        const status_type st = view().find(key_in, h, group, probing_length, join);
+        const status_type st = state().find(key_in, h, group, probing_length, join);
         if (!st.has_any()) value_store_.for_each(f, h, group);
         return st;
     }
@@ -866,7 +1247,7 @@ public:
                                 index_type probing_length = defaults::probing_length()) const noexcept {
         warpcore::detail::ImmediateJoin join{hash_table_.status_};
         handle_type h{0};
-        const status_type st = view().find(key_in, h, group, probing_length, join);
+        const status_type st = state().find(key_in, h, group, probing_length, join);
         num_out = st.has_any() ? 0 : h.value_count();
         return st;
     }
@@ -881,48 +1262,106 @@ public:
         if (!hash_table_.is_initialized_ || num_in == 0) return;
         using key_view = typename hash_table_type::view_type;
         using key_core = detail::BucketListKeyCore<key_view, typename value_store_type::view_type>;
+        // in chunks of the table's scratch, large batches grouped by key first
         if constexpr (warpcore::detail::fixed_step_scheme<typename key_view::probing_scheme_type>::value &&
                       warpcore::detail::owner_insert_capable<key_core>()) {
-            // key pass on the lane-owner kernel, then one lane per pair appends
-            // (in chunks of the table's scratch: each pair's slot and key status)
-            constexpr index_type chunk = index_type(1) << 24;
-            const index_type cap = num_in < chunk ? num_in : chunk;
             // (slot indices below detail::kSlotAppendFailed fit slot_of)
             if (warpcore::detail::owner_inserts() && hash_table_.capacity() < index_type(detail::kSlotAppendFailed) &&
-                reserve_scratch(cap)) {
+                reserve_scratch(std::min(num_in, insert_chunk))) {
                 constexpr bool statuses = !std::is_same<StatusHandler, status_handlers::ReturnNothing>::value;
-                std::uint32_t* slot_of = scratch_;
-                Status* key_status = reinterpret_cast<Status*>(scratch_ + scratch_cap_);
-                for (index_type first = 0; first < num_in; first += cap) {
-                    const index_type n = num_in - first < cap ? num_in - first : cap;
-                    storage::kernels::fill<std::uint32_t>
-                        <<<warpcore::detail::grid_for(n, 1, 8), block_size(), 0, stream>>>(slot_of, n, ~0u);
-                    const key_core core{hash_table_.view(), slot_of, values_in + first, value_store_.view(),
-                                        max_values_per_key_};
-                    Status* ks = statuses && status_out != nullptr ? key_status : nullptr;
-                    if (ks != nullptr)
-                        warpcore::detail::launch_insert_owner<key_core, status_handlers::ReturnStatus, false>(
-                            keys_in + first, nullptr, n, core, probing_length, ks, stream, nullptr);
-                    else
-                        warpcore::detail::launch_insert_owner<key_core, status_handlers::ReturnNothing, false>(
-                            keys_in + first, nullptr, n, core, probing_length, nullptr, stream, nullptr);
+                const bool wanted = statuses && status_out != nullptr;
+                warpcore::detail::MutationTracker::Exclusive exclusive(hash_table_.mutations_, stream);
+                index_type done = 0;
+                if (!wanted && exclusive.granted())
+                    done = insert_grouped(keys_in, values_in, num_in, stream, probing_length);
+                if (done != 0) exclusive.use();
+                if (done < num_in) {
                     typename StatusHandler::base_type* out = nullptr;
                     if constexpr (statuses)
-                        if (status_out != nullptr) out = status_out + first;
-                    kernels::bl_append<view_type, StatusHandler>
-                        <<<warpcore::detail::grid_for(n, 1, 32), block_size(), 0, stream>>>(
-                            values_in + first, n, slot_of, ks, view(), out);
+                        if (wanted) out = status_out + done;
+                    insert_passes<StatusHandler>(keys_in + done, values_in + done, num_in - done, stream,
+                                                 probing_length, out, nullptr);
                 }
                 if (stream == 0) (void)hipStreamSynchronize(stream);
                 return;
             }
         }
+        hash_table_.mutations_.note(stream);
         kernels::bl_insert<view_type, StatusHandler>
             <<<warpcore::detail::grid_for(num_in, cg_size()), block_size(), 0, stream>>>(
-                keys_in, values_in, num_in, view(), probing_length, status_out);
+                keys_in, values_in, num_in, state(), probing_length, status_out);
         if (stream == 0) (void)hipStreamSynchronize(stream);
     }
 
+private:
+    static constexpr index_type insert_chunk = index_type(1) << 24;
+
+    // The general insert: the key pass on the lane-owner kernel, then one lane
+    // per pair appends, in chunks of the table's scratch (each pair's slot and
+    // key status). With num_dev the batch is used when *num_dev is not 0.
+    template<class StatusHandler>
+    WC_H void insert_passes(const key_type* keys_in, const value_type* values_in, index_type num_in,
+                            hipStream_t stream, index_type probing_length,
+                            typename StatusHandler::base_type* status_out, const index_type* num_dev) noexcept {
+        using key_core = detail::BucketListKeyCore<typename hash_table_type::view_type,
+                                                   typename value_store_type::view_type>;
+        constexpr bool statuses = !std::is_same<StatusHandler, status_handlers::ReturnNothing>::value;
+        const index_type cap = std::min(num_in, insert_chunk);
+        std::uint32_t* slot_of = scratch_;
+        Status* key_status = reinterpret_cast<Status*>(scratch_ + scratch_cap_);
+        for (index_type first = 0; first < num_in; first += cap) {
+            const index_type n = num_in - first < cap ? num_in - first : cap;
+            kernels::bl_clear<<<warpcore::detail::grid_for(n, 1, 8), block_size(), 0, stream>>>(slot_of, n, num_dev);
+            const key_core core{hash_table_.state(), slot_of, values_in + first, value_store_.view(),
+                                max_values_per_key_};
+            Status* ks = statuses && status_out != nullptr ? key_status : nullptr;
+            if (ks != nullptr)
+                warpcore::detail::launch_insert_owner<key_core, status_handlers::ReturnStatus, false>(
+                    keys_in + first, nullptr, n, core, probing_length, ks, stream, num_dev);
+            else
+                warpcore::detail::launch_insert_owner<key_core, status_handlers::ReturnNothing, false>(
+                    keys_in + first, nullptr, n, core, probing_length, nullptr, stream, num_dev);
+            typename StatusHandler::base_type* out = nullptr;
+            if constexpr (statuses)
+                if (status_out != nullptr) out = status_out + first;
+            kernels::bl_append<view_type, StatusHandler>
+                <<<warpcore::detail::grid_for(n, 1, 32), block_size(), 0, stream>>>(values_in + first, n, slot_of, ks,
+                                                                                    state(), out, num_dev);
+        }
+    }
+
+    WC_HD view_type state() const noexcept {
+        return view_type{hash_table_.state(), value_store_.view(), max_values_per_key_};
+    }
+
+    // Large batches without statuses, grouped by key within table regions,
+    // where nothing else modifies the key table meanwhile; the number of
+    // pairs taken (the rest is the general insert's).
+    WC_H index_type insert_grouped(const key_type* keys_in, const value_type* values_in, index_type num_in,
+                                   hipStream_t stream, index_type probing_length) noexcept {
+        using key_view = typename hash_table_type::view_type;
+        using core_type = detail::BucketListGroupCore<key_view, typename value_store_type::view_type>;
+        using pair_type = detail::PairRecord<key_type, value_type>;
+        const key_view keys = hash_table_.state();
+        const core_type core{keys, value_store_.view(), max_values_per_key_};
+        index_type done = 0;
+        while (done < num_in) {
+            const index_type n = std::min(num_in - done, warpcore::detail::kPartChunk);
+            if (!warpcore::detail::groups_pay<pair_type>(n, keys.geometry(), stream)) break;
+            const key_type* k = keys_in + done;
+            const value_type* v = values_in + done;
+            if (!warpcore::detail::insert_grouped(k, v, n, core, keys, probing_length, stream,
+                                                  [&](const index_type* count) {
+                                                      insert_passes<status_handlers::ReturnNothing>(
+                                                          k, v, n, stream, probing_length, nullptr, count);
+                                                  }))
+                break;
+            done += n;
+        }
+        return done;
+    }
+
+public:
     // :333-424, the same two passes as MultiValueHashTable::retrieve
     template<class StatusHandler = defaults::status_handler_t>
     WC_H void retrieve(const key_type* keys_in, index_type num_in, index_type* begin_offsets_out,
@@ -958,7 +1397,7 @@ public:
                 begin_offsets_out, end_offsets_out, num_in);
             kernels::bl_retrieve<view_type, StatusHandler>
                 <<<warpcore::detail::grid_for(num_in, cg_size()), block_size(), 0, stream>>>(
-                    keys_in, num_in, begin_offsets_out, end_offsets_out, values_out, view(), probing_length,
+                    keys_in, num_in, begin_offsets_out, end_offsets_out, values_out, state(), probing_length,
                     status_out);
         } else {
             if (status_out != nullptr)
@@ -985,13 +1424,13 @@ public:
         storage::kernels::fill<index_type><<<warpcore::detail::grid_for(num_in, 1, 8), block_size(), 0, stream>>>(
             begin_offsets_out, num_in, index_type(0));
         warpcore::detail::launch_retrieve_owner<typename hash_table_type::view_type, StatusHandler>(
-            keys_in, num_in, reinterpret_cast<handle_type*>(begin_offsets_out), hash_table_.view(), probing_length,
+            keys_in, num_in, reinterpret_cast<handle_type*>(begin_offsets_out), hash_table_.state(), probing_length,
             status_out, stream);
         kernels::bl_counts<handle_type><<<warpcore::detail::grid_for(num_in, 1, 8), block_size(), 0, stream>>>(
             reinterpret_cast<const std::uint64_t*>(begin_offsets_out), num_in, end_offsets_out);
         warpcore::detail::device_scan(end_offsets_out, end_offsets_out, num_in, scan_parts_, true, stream);
         kernels::bl_walk<view_type><<<warpcore::detail::grid_for(num_in, 1, 32), block_size(), 0, stream>>>(
-            num_in, begin_offsets_out, end_offsets_out, values_out, view());
+            num_in, begin_offsets_out, end_offsets_out, values_out, state());
         num_out = 0;
         (void)hipMemcpyAsync(&num_out, end_offsets_out + (num_in - 1), sizeof(index_type), hipMemcpyDeviceToHost,
                              stream);
@@ -1020,7 +1459,7 @@ public:
         (void)hipMemsetAsync(tmp, 0, sizeof(index_type), stream);
         kernels::retrieve_all<typename hash_table_type::view_type>
             <<<warpcore::detail::grid_for(key_capacity(), 1, 8), block_size(), 0, stream>>>(
-                keys_out, static_cast<handle_type*>(nullptr), tmp, hash_table_.view());
+                keys_out, static_cast<handle_type*>(nullptr), tmp, hash_table_.state());
         (void)hipMemcpyAsync(&num_out, tmp, sizeof(index_type), hipMemcpyDeviceToHost, stream);
         (void)hipStreamSynchronize(stream);
     }
@@ -1038,7 +1477,7 @@ public:
         if (num_in != 0)
             kernels::bl_num_values<view_type, StatusHandler>
                 <<<warpcore::detail::grid_for(num_in, cg_size()), block_size(), 0, stream>>>(
-                    keys_in, num_in, tmp, num_per_key_out, view(), probing_length, status_out);
+                    keys_in, num_in, tmp, num_per_key_out, state(), probing_length, status_out);
         (void)hipMemcpyAsync(&num_out, tmp, sizeof(index_type), hipMemcpyDeviceToHost, stream);
         (void)hipStreamSynchronize(stream);
     }
@@ -1049,7 +1488,7 @@ public:
         index_type* tmp = hash_table_.temp_.get();
         (void)hipMemsetAsync(tmp, 0, sizeof(index_type), stream);
         kernels::bl_total_values<view_type>
-            <<<warpcore::detail::grid_for(key_capacity(), 1, 8), block_size(), 0, stream>>>(tmp, view());
+            <<<warpcore::detail::grid_for(key_capacity(), 1, 8), block_size(), 0, stream>>>(tmp, state());
         index_type out = 0;
         (void)hipMemcpyAsync(&out, tmp, sizeof(index_type), hipMemcpyDeviceToHost, stream);
         (void)hipStreamSynchronize(stream);
@@ -1084,6 +1523,7 @@ public:
     WC_HD index_type max_values_per_key() const noexcept { return max_values_per_key_; }
     WC_HD bool is_copy() const noexcept { return is_copy_; }
 
+    // device state for a caller's kernels, which may modify the table at any time
     WC_HD view_type view() const noexcept {
         return view_type{hash_table_.view(), value_store_.view(), max_values_per_key_};
     }

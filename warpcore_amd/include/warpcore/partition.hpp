@@ -123,20 +123,20 @@ struct PartPlan {
     index_t a = 0, a_idx = 0, b = 0, b_idx = 0, spill = 0, c1 = 0, c2 = 0, left = 0, lists = 0, skewed = 0, bytes = 0;
     index_t counter_words = 0;
 
-    bool two_pass() const noexcept { return p2log != 0; }
+    WC_HD bool two_pass() const noexcept { return p2log != 0; }
 };
 
-// mean of a Poisson-like count to a segment size: six standard deviations
-WC_H unsigned part_capacity(double mean) noexcept {
-    const double c = mean + 6.0 * std::sqrt(mean) + 32.0;
+// mean of a Poisson-like count to a segment size: `sigmas` standard deviations
+WC_H unsigned part_capacity(double mean, double sigmas = 6.0) noexcept {
+    const double c = mean + sigmas * std::sqrt(mean) + 32.0;
     return unsigned((index_t(c) + 31) / 32 * 32);
 }
 
 template<class Core, class Rec, bool Idx>
-WC_H PartPlan make_part_plan(index_t n, const probing_schemes::Geometry& geo) noexcept {
+WC_H PartPlan make_part_plan(index_t n, const probing_schemes::Geometry& geo, unsigned rw = region_windows<Core>(),
+                             double sigmas = 6.0) noexcept {
     PartPlan p;
     p.n = n;
-    constexpr unsigned rw = region_windows<Core>();
     while ((1u << p.shift) < rw) ++p.shift;
     const index_t regions = SDIV(geo.windows, index_t(rw));
     if (regions > index_t(kOnePassRegions) * 256) return PartPlan{};
@@ -150,7 +150,7 @@ WC_H PartPlan make_part_plan(index_t n, const probing_schemes::Geometry& geo) no
     const double share = double(SDIV(SDIV(n, index_t(p.tile)), kPartXcds) * p.tile);   // records of one XCD
     const double per_region = double(rw) / double(geo.windows);
     const double f1 = std::min(1.0, per_region * double(index_t(1) << p.p2log));
-    p.cap1 = part_capacity(std::min(share, double(n)) * f1);
+    p.cap1 = part_capacity(std::min(share, double(n)) * f1, sigmas);
     const index_t rec = sizeof(Rec) + (Idx ? 4 : 0);
     auto place = [&](index_t& at, index_t bytes) {
         at = p.bytes;
@@ -159,7 +159,7 @@ WC_H PartPlan make_part_plan(index_t n, const probing_schemes::Geometry& geo) no
     const index_t a_records = index_t(p.buckets) * kPartXcds * p.cap1;
     index_t b_records;
     if (p.two_pass()) {
-        p.cap2 = part_capacity(double(n) * std::min(1.0, per_region)) + region_slack<Core>();
+        p.cap2 = part_capacity(double(n) * std::min(1.0, per_region), sigmas) + region_slack<Core>();
         p.tiles = unsigned(SDIV(index_t(p.cap1), index_t(p.tile)));
         const index_t bucket_bytes = (index_t(1) << p.p2log) * p.cap2 * rec;
         index_t gb = kRefineBytes / bucket_bytes / kPartXcds * kPartXcds;   // every XCD gets as many buckets
