@@ -92,6 +92,14 @@ def kernel_family(lib, op: str) -> str:
     return "retrieve_lockstep" if k & 2 else "retrieve_batched"
 
 
+def bulk_family(lib, op: str, n: int) -> str:
+    """The same for a call of n keys that fill most of an empty table: such
+    inserts of at least 2^20 keys run the region passes (part_scatter,
+    part_refine, part_build, part_tail), not the lane-owner kernel alone."""
+    family = kernel_family(lib, op)
+    return "insert_partitioned" if family == "insert_owner" and n >= 1 << 20 else family
+
+
 def probes_lib():
     """ctypes handle of warpcore_amd/probes/libwarpcore_probes.so, prototypes
     from its header."""
@@ -775,7 +783,7 @@ def main():
     achieved = per_op[dom] * n / (kt[dom] * 1e-3) / 1e9
     other = "retrieve" if dom == "insert" else "insert"
     achieved_other = per_op[other] * n / (kt[other] * 1e-3) / 1e9
-    fam = {op: kernel_family(g.lib, op) for op in ("insert", "retrieve")}
+    fam = {op: bulk_family(g.lib, op, n) for op in ("insert", "retrieve")}
     roofline = {"bound": "hbm", "kernel": f"{fam[dom]} [SVHT u64/u64 cg 8]", "achieved": round(achieved, 1),
                 "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                 "traffic": read_traffic(fam[dom], args.log2_keys),
@@ -787,7 +795,8 @@ def main():
                                  "traffic": read_traffic(fam[other], args.log2_keys)}}
     # practical ceiling for random whole lines at the headline table's size
     lr = run_line_roofline(g, r64["table_bytes"], claim=True)
-    # inserts against the read-then-claim rate (one window and one CAS per key at best)
+    # inserts against the read-then-claim rate, one window and one CAS per key (region passes write
+    # windows back whole and can exceed it)
     lr["insert_vs_claim"] = round(n / (kt["insert"] * 1e-3) / 1e9 / lr["claim_glines_s"], 4)
     for op in ("retrieve", "insert"):
         tr = read_traffic(fam[op], args.log2_keys)
