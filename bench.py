@@ -57,6 +57,13 @@ def algorithmic_bytes(op: str, kb: int, vb: int) -> int:
     raise ValueError(op)
 
 
+def region_bytes(rec: int, table_bytes: int, n: int, passes: int) -> int:
+    """Bytes per key of an insert sorted by table region: records of `rec`
+    bytes read, written and read once more by each sorting pass, the table
+    streamed in and out."""
+    return round(rec * (1 + 2 * passes) + 2 * table_bytes / n)
+
+
 # Revision of the probing kernels' code; a traffic figure measured on
 # another revision is not used.
 KERNEL_REVISION = "owner-4"
@@ -509,7 +516,7 @@ def run_hashset(g: Gpu, log2n: int = 27, reps: int = 3):
     ok = ok and int(flags.sum()) == 0 and s.size(stream=g.stream) == n
     if not ok:
         raise RuntimeError("hash set result check failed")
-    res = {"capacity": s.capacity(), "cg": s.cg_size(), "insert": _rate(n, ins, 2 * LINE + 4),
+    res = {"capacity": s.capacity(), "cg": s.cg_size(), "insert": _rate(n, ins, region_bytes(4, 4 * s.capacity(), n, 2)),
            "contains_hits": _rate(n, hit, LINE + 4 + 1), "contains_misses": _rate(n, miss, LINE + 4 + 1)}
     del s, keys, absent, flags
     torch.cuda.empty_cache()
@@ -539,7 +546,8 @@ def run_bloom(g: Gpu, log2_bits: int = 30, k: int = 8, log2n: int = 27, reps: in
     bf.retrieve(absent, flags[:half], stream=g.stream)
     g.stream.synchronize()
     fpr = float(flags[:half].float().mean())
-    res = {"bytes": bf.bytes_total(), "cg": bf.cg_size(), "insert": _rate(n, ins, 2 * LINE + 8),
+    res = {"bytes": bf.bytes_total(), "cg": bf.cg_size(),
+           "insert": _rate(n, ins, region_bytes(8, bf.bytes_total(), n, 1)),
            "query": _rate(n, qry, LINE + 8 + 1), "fpr_measured": round(fpr, 5), "fpr_model": round(bf.fpr(n), 5)}
     del bf, keys, absent, queries, flags
     torch.cuda.empty_cache()
@@ -778,12 +786,14 @@ def main():
 
     n = r64["n"]
     per_op = {"insert": algorithmic_bytes("insert", 64, 64), "retrieve": algorithmic_bytes("retrieve", 64, 64)}
+    fam = {op: bulk_family(g.lib, op, n) for op in ("insert", "retrieve")}
+    if fam["insert"] == "insert_partitioned":
+        per_op["insert"] = region_bytes(16, r64["table_bytes"], n, 2)
     kt = {"insert": r64["insert_ms"], "retrieve": r64["retrieve_ms"]}
     dom = max(kt, key=kt.get)
     achieved = per_op[dom] * n / (kt[dom] * 1e-3) / 1e9
     other = "retrieve" if dom == "insert" else "insert"
     achieved_other = per_op[other] * n / (kt[other] * 1e-3) / 1e9
-    fam = {op: bulk_family(g.lib, op, n) for op in ("insert", "retrieve")}
     roofline = {"bound": "hbm", "kernel": f"{fam[dom]} [SVHT u64/u64 cg 8]", "achieved": round(achieved, 1),
                 "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                 "traffic": read_traffic(fam[dom], args.log2_keys),
