@@ -194,6 +194,45 @@ def test_full_bucketlist_multisets(cuda):
     assert torch.equal(a, b)
 
 
+def test_full_bucketlist_grouped_equals_pair_by_pair(cuda):
+    """Inserts without statuses, which group the pairs by key, against inserts
+    with statuses, which append them one by one: 2^26 pairs whose
+    multiplicities are geometric (mean 8), drawn with whole numbers so that
+    the seed alone determines them. Same offsets, same (key, value) multisets,
+    same cells used, on a first pass and after another table's pass between."""
+    from warpcore_amd.tables import BucketListHashTable
+    n, d = 1 << 26, 1 << 23
+    print("[full] bucketlist u32 2^26 pairs, grouped and pair by pair", flush=True)
+    ukeys = _gen_unique(d, 32, 0x7000)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(0xC8)
+    u = torch.rand(d, device="cuda", dtype=torch.float64, generator=gen)
+    weight = (-torch.log1p(-u) * (1 << 20)).to(torch.int64) + 1
+    upto = torch.cumsum(weight, 0)   # exact in any order of the additions
+    pick = torch.searchsorted(upto, torch.randint(0, int(upto[-1]), (n,), device="cuda", generator=gen), right=True)
+    dk, dv = ukeys[pick].contiguous(), _gen_uniform(n, 32, 0xC9)
+    del u, weight, upto
+    count = torch.bincount(pick, minlength=d)
+    other = BucketListHashTable(math.ceil(d / 0.9), 5 * n // 2, 32, 32, grow_factor=1.1, min_bucket_size=1)
+    pack = lambda k, v: (k.to(torch.int64) & 0xFFFFFFFF) << 32 | (v.to(torch.int64) & 0xFFFFFFFF)
+    want = torch.sort(pack(dk, dv)).values
+    st = torch.empty(n, dtype=torch.int32, device="cuda")
+    cells = []
+    for statuses in (st, None, None):
+        t = BucketListHashTable(math.ceil(d / 0.9), 5 * n // 2, 32, 32, grow_factor=1.1, min_bucket_size=1)
+        t.insert(dk, dv, status_out=statuses)
+        other.init()
+        other.insert(dk.flip(0), dv)
+        beg, end = (torch.zeros(d, dtype=torch.int64, device="cuda") for _ in range(2))
+        out = torch.zeros(n, dtype=torch.int32, device="cuda")
+        assert t.retrieve(ukeys, beg, end, out) == n
+        assert torch.equal(end, torch.cumsum(count, 0)) and torch.equal(end - beg, count)
+        owner = torch.repeat_interleave(ukeys, count)
+        assert torch.equal(torch.sort(pack(owner, out)).values, want)
+        cells.append(t.value_cells_used())
+    assert cells[0] == cells[1] == cells[2]
+
+
 def test_full_hashset_u32(cuda):
     from warpcore_amd.tables import HashSet
     n = 1 << 27
