@@ -188,3 +188,18 @@ def test_counting_combined_add_saturates(dlib, max_count, preset):
     assert np.all(got_c[is_hot] == min(preset + int(is_hot.sum()), max_count))
     assert np.all(got_c[~is_hot] == 1)
     assert word.value == S_DUP                        # duplicate_key joined, no index_overflow (64)
+
+
+def test_inserts_from_threads_on_their_own_null_stream(cuda):
+    """The null stream of a translation unit built with
+    -fgpu-default-stream=per-thread is another one in every host thread:
+    batches large enough for the region passes, none waited for."""
+    lib = ctypes.CDLL(str(LIB.with_name("libwc_per_thread.so")))
+    lib.wcp_insert_from_threads.restype = ctypes.c_uint64
+    lib.wcp_insert_from_threads.argtypes = [ctypes.c_void_p] + [ctypes.c_uint64] * 3 + [ctypes.c_void_p]
+    n = 6_000_003   # each half more than 3/8 of the slots
+    keys = unique_keys(n, 64, seed=31)
+    kd, out = to_dev(keys), dev_empty(n, 64, 0x55)
+    torch.cuda.synchronize()
+    assert lib.wcp_insert_from_threads(_p(kd), n, 2, int(n / 0.85), _p(out)) == n
+    assert torch.equal(out, kd)

@@ -8,10 +8,10 @@
 // - Every bulk call that modifies the table notes its stream. A call may run
 //   exclusively while all of them used that one stream, which then orders
 //   them. A second stream, a call under capture (its graph may be replayed at
-//   any time), the per-thread default stream (one handle, many streams), and
-//   a copy or a view of the table handed out (user kernels may modify the
-//   table through the device calls) end that; the calls that follow use the
-//   compare-and-swap paths.
+//   any time), a handle of the per-thread default stream (one handle, many
+//   streams: per_thread_stream), and a copy or a view of the table handed out
+//   (user kernels may modify the table through the device calls) end that;
+//   the calls that follow use the compare-and-swap paths.
 // - An exclusive call leaves an event behind its kernels. A later modifying
 //   call on another stream waits for it on the device, and handing out a copy
 //   or a view, or noting a call under capture, waits for it on the host.
@@ -27,6 +27,16 @@
 
 namespace warpcore {
 namespace detail {
+
+// Whether a handle names another stream in every host thread: the per-thread
+// handle, and the null handle where launches on it go to the calling thread's
+// own stream (-fgpu-default-stream=per-thread).
+WC_H bool per_thread_stream(hipStream_t stream) noexcept {
+#if defined(HIP_API_PER_THREAD_DEFAULT_STREAM)
+    if (stream == nullptr) return true;
+#endif
+    return stream == hipStreamPerThread;
+}
 
 class MutationTracker {
     struct State {
@@ -135,7 +145,7 @@ private:
             return false;
         }
         if (s_->fenced && s_->fence_stream != stream) (void)hipStreamWaitEvent(stream, s_->fence, 0);
-        if (stream == hipStreamPerThread || (s_->any && s_->stream != stream)) s_->mixed = true;
+        if (per_thread_stream(stream) || (s_->any && s_->stream != stream)) s_->mixed = true;
         s_->any = true;
         s_->stream = stream;
         return !s_->mixed && !s_->shared;
