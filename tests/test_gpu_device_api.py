@@ -203,3 +203,29 @@ def test_inserts_from_threads_on_their_own_null_stream(cuda):
     torch.cuda.synchronize()
     assert lib.wcp_insert_from_threads(_p(kd), n, 2, int(n / 0.85), _p(out)) == n
     assert torch.equal(out, kd)
+
+
+@pytest.fixture(scope="module")
+def vlib(cuda):
+    lib = ctypes.CDLL(str(LIB.with_name("libwc_value_types.so")))
+    for f in (lib.wcv_single, lib.wcv_lists):
+        f.restype = ctypes.c_int64
+        f.argtypes = [ctypes.c_int, ctypes.c_void_p, ctypes.c_uint64, ctypes.c_uint64]
+    return lib
+
+
+@pytest.mark.parametrize("kind,bits", [(0, 64), (1, 64), (2, 32)])
+def test_single_values_of_several_words(vlib, kind, bits):
+    """32, 16 and 12 bytes: only the last one's slots fit the region passes' records."""
+    n = 3_000_001
+    kd = to_dev(unique_keys(n, bits, seed=41 + kind))
+    torch.cuda.synchronize()
+    assert vlib.wcv_single(kind, _p(kd), n, int(n / 0.9)) == 0
+
+
+@pytest.mark.parametrize("kind,bits", [(0, 64), (1, 64), (2, 32), (3, 32)])
+def test_lists_of_values_of_several_words(vlib, kind, bits):
+    n = 1_200_001
+    kd = to_dev(unique_keys(n, bits, seed=51 + kind))
+    torch.cuda.synchronize()
+    assert vlib.wcv_lists(kind, _p(kd), n, int(n / 0.9)) == 0

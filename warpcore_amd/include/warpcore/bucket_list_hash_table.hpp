@@ -1272,8 +1272,9 @@ public:
                 const bool wanted = statuses && status_out != nullptr;
                 warpcore::detail::MutationTracker::Exclusive exclusive(hash_table_.mutations_, stream);
                 index_type done = 0;
-                if (!wanted && exclusive.granted())
-                    done = insert_grouped(keys_in, values_in, num_in, stream, probing_length);
+                if constexpr (warpcore::detail::part_record<warpcore::detail::PairRecord<key_type, value_type>>())
+                    if (!wanted && exclusive.granted())
+                        done = insert_grouped(keys_in, values_in, num_in, stream, probing_length);
                 if (done != 0) exclusive.use();
                 if (done < num_in) {
                     typename StatusHandler::base_type* out = nullptr;

@@ -838,11 +838,19 @@ struct has_region_op : std::false_type {};
 template<class Core>
 struct has_region_op<Core, std::void_t<decltype(Core::region_op)>> : std::true_type {};
 
+// Records that the sorting tiles hold in LDS: up to 16 bytes (a tile of them
+// takes 80 KB, two blocks per CU; of 24 bytes 112 KB, half the wavefronts, of
+// 32 bytes 176 KB, more than a CU has), and plain enough for shared memory.
+template<class Rec>
+constexpr bool part_record() noexcept {
+    return sizeof(Rec) <= 16 && std::is_trivially_default_constructible<Rec>::value;
+}
+
 // Windows of 4..16 slots with a fixed step, at most 64 KB a region.
-template<class Core>
+template<class Core, class Rec>
 constexpr bool partition_capable() noexcept {
     return has_region_op<Core>::value && fixed_step_scheme<typename Core::probing_scheme_type>::value &&
-           Core::cg_size() >= 4 && Core::cg_size() <= 16;
+           Core::cg_size() >= 4 && Core::cg_size() <= 16 && part_record<Rec>();
 }
 
 // Grid of a launch whose blocks are dealt to the XCDs in turn: a multiple of
