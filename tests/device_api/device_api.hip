@@ -101,6 +101,15 @@ __global__ void bucketlist_roundtrip(const typename Table::key_type* keys, const
     if (group.thread_rank() == 0) status_out[gid] = st.base();
 }
 
+// A status handler that counts its calls per key.
+struct CountCalls {
+    using base_type = std::uint32_t;
+    using tag = tags::status_handler;
+    WC_D static void handle(Status, base_type* out, index_t index) noexcept {
+        if (out != nullptr) atomicAdd(out + index, 1u);
+    }
+};
+
 unsigned blocks_for(index_t threads) { return unsigned((threads + 255) / 256); }
 
 // Both boolean status handlers, for one compile-time Ignore word.
@@ -367,6 +376,20 @@ int wcx_counting_u32_saturation(const std::uint32_t* keys, std::uint64_t n, std:
                                                           reinterpret_cast<Status*>(status_out));
     table.retrieve(keys, n, counts_out);
     *table_status = table.peek_status().base();
+    return int(hipDeviceSynchronize());
+}
+
+// Calls of a status handler per key (calls_out, zeroed by the caller) of one
+// bulk insert into a SingleValueHashTable (which 0) or a HashSet (1).
+int wcx_handler_calls(int which, const std::uint64_t* keys, std::uint64_t n, std::uint64_t capacity,
+                      std::uint32_t* calls_out) {
+    if (which == 0) {
+        SingleValueHashTable<std::uint64_t, std::uint64_t> table(capacity);
+        table.insert<CountCalls>(keys, keys, n, 0, defaults::probing_length(), calls_out);
+        return int(hipDeviceSynchronize());
+    }
+    HashSet<std::uint64_t> set(capacity);
+    set.insert<CountCalls>(keys, n, 0, defaults::probing_length(), calls_out);
     return int(hipDeviceSynchronize());
 }
 

@@ -229,3 +229,17 @@ def test_lists_of_values_of_several_words(vlib, kind, bits):
     kd = to_dev(unique_keys(n, bits, seed=51 + kind))
     torch.cuda.synchronize()
     assert vlib.wcv_lists(kind, _p(kd), n, int(n / 0.9)) == 0
+
+
+@pytest.mark.parametrize("which", [0, 1])
+def test_status_handler_runs_once_per_key(dlib, which):
+    """A batch large enough for the region passes, with duplicates and invalid keys."""
+    dlib.wcx_handler_calls.argtypes = [ctypes.c_int, ctypes.c_void_p, ctypes.c_uint64, ctypes.c_uint64, ctypes.c_void_p]
+    n = 3_000_001
+    keys = unique_keys(n, 64, seed=61)
+    keys[5::5] = keys[1::5]
+    keys[::1009] = 0
+    kd, calls = to_dev(keys), torch.zeros(n, dtype=torch.int32, device="cuda")
+    torch.cuda.synchronize()
+    assert dlib.wcx_handler_calls(which, _p(kd), n, int(n / 0.9), _p(calls)) == 0
+    assert bool((calls == 1).all())

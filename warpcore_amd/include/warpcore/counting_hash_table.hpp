@@ -727,7 +727,8 @@ private:
     template<class StatusHandler>
     WC_H bool partition_entries(const CombineBuffers& buf, index_type n, hipStream_t stream, index_type probing_length,
                                 typename StatusHandler::base_type* status_out) noexcept {
-        if constexpr (detail::partition_capable<add_view_type, typename base_type::slot_type>() &&
+        if constexpr (detail::partition_capable<add_view_type, typename base_type::slot_type,
+                                                status_handlers::ReturnStatus>() &&
                       sizeof(value_type) == 8) {
             if (max_count_ == std::numeric_limits<value_type>::max() && detail::refill_inserts() &&
                 detail::owner_inserts() && n / 4 >= (index_type(1) << 20) && n / 4 >= capacity() / 8 * 3) {

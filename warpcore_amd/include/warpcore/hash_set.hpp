@@ -233,7 +233,7 @@ public:
                      typename StatusHandler::base_type* status_out = nullptr) noexcept {
         static_assert(checks::is_status_handler<StatusHandler>(), "not a valid status handler type");
         if (!is_initialized_ || num_in == 0) return;
-        if constexpr (detail::partition_capable<view_type, key_type>()) {
+        if constexpr (detail::partition_capable<view_type, key_type, StatusHandler>()) {
             const bool* values = nullptr;
             if (detail::insert_partitioned_first<view_type, StatusHandler, false, key_type>(
                     mutations_, keys_in, values, num_in, state(), probing_length, status_out, stream,

@@ -846,11 +846,13 @@ constexpr bool part_record() noexcept {
     return sizeof(Rec) <= 16 && std::is_trivially_default_constructible<Rec>::value;
 }
 
-// Windows of 4..16 slots with a fixed step, at most 64 KB a region.
-template<class Core, class Rec>
+// Windows of 4..16 slots with a fixed step, at most 64 KB a region; handlers
+// that may run twice per key.
+template<class Core, class Rec, class StatusHandler>
 constexpr bool partition_capable() noexcept {
     return has_region_op<Core>::value && fixed_step_scheme<typename Core::probing_scheme_type>::value &&
-           Core::cg_size() >= 4 && Core::cg_size() <= 16 && part_record<Rec>();
+           Core::cg_size() >= 4 && Core::cg_size() <= 16 && part_record<Rec>() &&
+           status_handlers::overwrites<StatusHandler>::value;
 }
 
 // Grid of a launch whose blocks are dealt to the XCDs in turn: a multiple of

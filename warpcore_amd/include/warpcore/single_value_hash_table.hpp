@@ -542,7 +542,7 @@ public:
                      typename StatusHandler::base_type* status_out = nullptr) noexcept {
         static_assert(checks::is_status_handler<StatusHandler>(), "not a valid status handler type");
         if (!is_initialized_ || num_in == 0) return;
-        if constexpr (!soa_storage && detail::partition_capable<view_type, slot_type>()) {
+        if constexpr (!soa_storage && detail::partition_capable<view_type, slot_type, StatusHandler>()) {
             if (detail::insert_partitioned_first<view_type, StatusHandler, true, slot_type>(
                     mutations_, keys_in, values_in, num_in, state(), probing_length, status_out, stream,
                     capacity() * sizeof(slot_type)))

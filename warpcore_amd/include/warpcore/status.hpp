@@ -193,6 +193,21 @@ public:
     }
 };
 
+// Whether a second handle() of a key leaves what it alone would have left.
+// The region inserts write `none` for the whole batch as they read it and the
+// other outcomes later, so they need that; any other handler (one that counts
+// or joins) runs in the general kernels, which call it once per key.
+template<class Handler>
+struct overwrites : std::false_type {};
+template<>
+struct overwrites<ReturnNothing> : std::true_type {};
+template<>
+struct overwrites<ReturnStatus> : std::true_type {};
+template<Status::base_type Ignore>
+struct overwrites<ReturnBoolean<Ignore>> : std::true_type {};
+template<Status::base_type Ignore>
+struct overwrites<ReturnAnyFlag<Ignore>> : std::true_type {};
+
 }  // namespace status_handlers
 
 }  // namespace warpcore
