@@ -1,7 +1,8 @@
 """Builds the test libraries of this folder (test infrastructure, gfx950, header-only library):
 libwc_device_api.so, user kernels that call the tables' device API,
-libwc_per_thread.so, host threads whose null stream is their own, and
-libwc_value_types.so, values of several words."""
+libwc_per_thread.so, host threads whose null stream is their own,
+libwc_value_types.so, values of several words, and libwc_host_memory.so, an
+operator new that throws."""
 from __future__ import annotations
 
 import concurrent.futures
@@ -11,7 +12,8 @@ from pathlib import Path
 
 HERE = Path(__file__).resolve().parent
 REPO = HERE.parents[1]
-SOURCES = {"device_api": [], "per_thread": ["-fgpu-default-stream=per-thread"], "value_types": []}   # and their own flags
+SOURCES = {"device_api": [], "per_thread": ["-fgpu-default-stream=per-thread"], "value_types": [],
+           "host_memory": ["-Wl,-Bsymbolic"]}   # and their own flags
 LIB = HERE / "libwc_device_api.so"
 
 

@@ -243,3 +243,16 @@ def test_status_handler_runs_once_per_key(dlib, which):
     torch.cuda.synchronize()
     assert dlib.wcx_handler_calls(which, _p(kd), n, int(n / 0.9), _p(calls)) == 0
     assert bool((calls == 1).all())
+
+
+def test_insert_without_host_memory(cuda):
+    """Nothing in a bulk insert depends on operator new: no exception leaves
+    it, and every key is stored."""
+    lib = ctypes.CDLL(str(LIB.with_name("libwc_host_memory.so")))
+    lib.wch_insert.restype = ctypes.c_uint64
+    lib.wch_insert.argtypes = [ctypes.c_void_p, ctypes.c_uint64, ctypes.c_uint64, ctypes.c_void_p]
+    n = 3_000_001
+    kd, out = to_dev(unique_keys(n, 64, seed=71)), dev_empty(n, 64, 0x55)
+    torch.cuda.synchronize()
+    assert lib.wch_insert(_p(kd), n, int(n / 0.9), _p(out)) == n
+    assert torch.equal(out, kd)

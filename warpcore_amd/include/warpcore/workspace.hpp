@@ -18,7 +18,7 @@
 #include "base.hpp"
 
 #include <mutex>
-#include <vector>
+#include <new>
 
 namespace warpcore {
 namespace detail {
@@ -29,7 +29,9 @@ constexpr std::size_t kWorkspaceUnit = std::size_t(1) << 20;   // leases are rou
 class WorkspacePool {
 public:
     static WorkspacePool& instance() noexcept {
-        static WorkspacePool* pool = new WorkspacePool;   // never destroyed: tables may outlive static objects
+        // never destroyed: tables may outlive static objects
+        alignas(WorkspacePool) static unsigned char place[sizeof(WorkspacePool)];
+        static WorkspacePool* pool = ::new (static_cast<void*>(place)) WorkspacePool;
         return *pool;
     }
 
@@ -39,6 +41,7 @@ public:
         int device = 0;
         hipEvent_t done = nullptr;   // behind the last user's kernels
         bool leased = false;
+        Buffer* next = nullptr;
     };
 
     WC_H void add_user() noexcept {
@@ -58,7 +61,7 @@ public:
         if (bytes > kWorkspaceLimit || hipGetDevice(&device) != hipSuccess) return nullptr;
         std::lock_guard<std::mutex> lock(mu_);
         Buffer* best = nullptr;
-        for (Buffer* b : buffers_)
+        for (Buffer* b = first_; b != nullptr; b = b->next)
             if (!b->leased && b->device == device && b->bytes >= bytes && (best == nullptr || b->bytes < best->bytes))
                 best = b;
         if (best != nullptr) {
@@ -69,15 +72,9 @@ public:
             best->leased = true;
             return best;
         }
-        std::size_t held = 0;
-        for (const Buffer* b : buffers_)
-            if (b->device == device) held += b->bytes;
-        if (held + bytes > kWorkspaceLimit) {
+        if (held_on(device) + bytes > kWorkspaceLimit) {
             free_idle(device);
-            held = 0;
-            for (const Buffer* b : buffers_)
-                if (b->device == device) held += b->bytes;
-            if (held + bytes > kWorkspaceLimit) return nullptr;
+            if (held_on(device) + bytes > kWorkspaceLimit) return nullptr;
         }
         Buffer* b = new (std::nothrow) Buffer;
         if (b == nullptr) return nullptr;
@@ -99,7 +96,8 @@ public:
             }
         }
         b->leased = true;
-        buffers_.push_back(b);
+        b->next = first_;
+        first_ = b;
         return b;
     }
     WC_H void release(Buffer* b, hipStream_t stream) noexcept {
@@ -114,31 +112,36 @@ public:
     // bytes held on all devices
     WC_H std::size_t bytes_held() noexcept {
         std::lock_guard<std::mutex> lock(mu_);
-        std::size_t held = 0;
-        for (const Buffer* b : buffers_) held += b->bytes;
-        return held;
+        return held_on(-1);
     }
 
 private:
+    // bytes of one device's buffers, or (-1) of all
+    WC_H std::size_t held_on(int device) const noexcept {
+        std::size_t held = 0;
+        for (const Buffer* b = first_; b != nullptr; b = b->next)
+            if (device < 0 || b->device == device) held += b->bytes;
+        return held;
+    }
     // frees the buffers not leased (of one device, or all); hipFree waits
     // for the kernels that still use one
     WC_H void free_idle(int device) noexcept {
-        std::size_t kept = 0;
-        for (Buffer* b : buffers_) {
+        for (Buffer** at = &first_; *at != nullptr;) {
+            Buffer* b = *at;
             if (b->leased || (device >= 0 && b->device != device)) {
-                buffers_[kept++] = b;
+                at = &b->next;
                 continue;
             }
+            *at = b->next;
             (void)hipEventSynchronize(b->done);
             (void)hipFree(b->p);
             (void)hipEventDestroy(b->done);
             delete b;
         }
-        buffers_.resize(kept);
     }
 
     std::mutex mu_;
-    std::vector<Buffer*> buffers_;
+    Buffer* first_ = nullptr;   // linked in the buffers themselves: a lease allocates nothing that may throw
     std::size_t users_ = 0;
 };
 
