@@ -160,6 +160,34 @@ def test_inserts_from_two_streams(cuda):
         assert torch.equal(out, vd)
 
 
+def test_insert_beside_a_capture_of_another_stream(cuda):
+    """A bulk insert whose workspace is allocated while another stream is
+    captured in the global mode: the insert runs, the capture stays valid."""
+    from warpcore_amd.tables import BloomFilter, SingleValueHashTable
+    n = 3_000_001
+    keys = unique_keys(n, 64, seed=23)
+    kd, vd = to_dev(keys), to_dev(_value_of(keys, 64))
+    t, bf = SingleValueHashTable(math.ceil(n / 0.85), 64, 64), BloomFilter(1 << 26, 4, 64)
+    x = torch.zeros(1024, device="cuda")
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    g = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g, stream=b, capture_error_mode="global"):
+        x.add_(1)
+        t.insert(kd, vd, stream=a)
+        bf.insert(kd, stream=a)
+        x.add_(2)
+    out, flags = torch.zeros_like(vd), torch.zeros(n, dtype=torch.uint8, device="cuda")
+    torch.cuda.synchronize()
+    t.retrieve(kd, out)
+    bf.retrieve(kd, flags)
+    assert torch.equal(out, vd) and bool((flags == 1).all()) and t.size() == n
+    for replay in range(3):
+        g.replay()
+        torch.cuda.synchronize()
+        assert bool((x == 3 * (replay + 1)).all())
+
+
 @pytest.mark.parametrize("kb,n,load,shape", [
     (32, 1 << 20, 0.9, "distinct"), (32, 16_000_003, 0.9, "repeats"),   # one pass and two
     (32, 3_000_001, 0.93, "hot"), (32, 16_000_003, 0.9, "few"),

@@ -131,6 +131,23 @@ WC_H unsigned grid_for_lanes(index_t items) noexcept {
     return unsigned(g == 0 ? 1 : g);
 }
 
+// While this object lives, calls of this thread that are not part of a stream
+// capture (allocations, host waits) neither fail nor end a capture that some
+// stream of the process has open in the global or thread-local mode.
+class RelaxedCapture {
+public:
+    WC_H RelaxedCapture() noexcept : exchanged_(hipThreadExchangeStreamCaptureMode(&mode_) == hipSuccess) {}
+    RelaxedCapture(const RelaxedCapture&) = delete;
+    RelaxedCapture& operator=(const RelaxedCapture&) = delete;
+    WC_H ~RelaxedCapture() noexcept {
+        if (exchanged_) (void)hipThreadExchangeStreamCaptureMode(&mode_);
+    }
+
+private:
+    hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;   // then the thread's own
+    bool exchanged_;
+};
+
 // Available device memory (hpc_helpers' available_gpu_memory).
 WC_H std::size_t available_gpu_memory() noexcept {
     std::size_t free_b = 0, total_b = 0;

@@ -128,12 +128,8 @@ private:
     WC_H void share_locked() const noexcept {
         s_->shared = true;
         if (!s_->fenced) return;
-        // also called while some stream of this thread is captured, where a
-        // host wait needs the relaxed mode
-        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-        const bool exchanged = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+        const RelaxedCapture relaxed;   // also called while some stream is captured
         (void)hipEventSynchronize(s_->fence);
-        if (exchanged) (void)hipThreadExchangeStreamCaptureMode(&mode);
         s_->fenced = false;
     }
     // whether `stream` orders every modification

@@ -12,7 +12,8 @@
 // or the device's memory would refuse a larger lease.
 //
 // Not for calls under stream capture: a graph would keep the buffer's address
-// beyond the lease.
+// beyond the lease. Beside a capture of another stream the pool allocates and
+// frees in the relaxed capture mode, so that the capture stays valid.
 #pragma once
 
 #include "base.hpp"
@@ -50,7 +51,9 @@ public:
     }
     WC_H void remove_user() noexcept {
         std::lock_guard<std::mutex> lock(mu_);
-        if (--users_ == 0) free_idle(-1);
+        if (--users_ != 0) return;
+        const RelaxedCapture relaxed;
+        free_idle(-1);
     }
 
     // a buffer of at least `bytes` on the current device, whose earlier use
@@ -60,6 +63,7 @@ public:
         int device = 0;
         if (bytes > kWorkspaceLimit || hipGetDevice(&device) != hipSuccess) return nullptr;
         std::lock_guard<std::mutex> lock(mu_);
+        const RelaxedCapture relaxed;
         Buffer* best = nullptr;
         for (Buffer* b = first_; b != nullptr; b = b->next)
             if (!b->leased && b->device == device && b->bytes >= bytes && (best == nullptr || b->bytes < best->bytes))
@@ -102,6 +106,7 @@ public:
     }
     WC_H void release(Buffer* b, hipStream_t stream) noexcept {
         std::lock_guard<std::mutex> lock(mu_);
+        const RelaxedCapture relaxed;
         if (hipEventRecord(b->done, stream) != hipSuccess) {
             (void)hipGetLastError();
             (void)hipStreamSynchronize(stream);   // no event to wait for: the kernels end here
