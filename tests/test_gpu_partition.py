@@ -188,6 +188,55 @@ def test_insert_beside_a_capture_of_another_stream(cuda):
         assert bool((x == 3 * (replay + 1)).all())
 
 
+def _streams_side_by_side():
+    """Two streams whose kernels do run beside each other (streams share a few
+    hardware queues)."""
+    x = torch.zeros(1024, device="cuda")
+    for _ in range(16):
+        a, b = torch.cuda.Stream(), torch.cuda.Stream()
+        after = torch.cuda.Event()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(a):
+            torch.cuda._sleep(20_000_000)
+            after.record(a)
+        with torch.cuda.stream(b):
+            x.add_(1)
+        b.synchronize()
+        beside = not after.query()
+        torch.cuda.synchronize()
+        if beside:
+            return a, b
+    pytest.skip("no two streams run beside each other")
+
+
+def test_insert_does_not_wait_for_another_stream(cuda):
+    """Stream a's insert is queued behind a long kernel; an insert into
+    another table on stream b ends before that kernel does."""
+    from warpcore_amd.tables import SingleValueHashTable
+    n = 3_000_001
+    keys = unique_keys(n, 64, seed=25)
+    kd, vd = to_dev(keys), to_dev(_value_of(keys, 64))
+    ta, tb = (SingleValueHashTable(math.ceil(n / 0.85), 64, 64) for _ in range(2))
+    a, b = _streams_side_by_side()
+    after = torch.cuda.Event()
+    ta.insert(kd, vd, stream=b)   # a workspace that both could use
+    ta.init(stream=b)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(a):
+        torch.cuda._sleep(1_000_000_000)   # some tenths of a second
+        after.record(a)
+    ta.insert(kd, vd, stream=a)
+    tb.insert(kd, vd, stream=b)
+    b.synchronize()
+    assert not after.query()   # the kernel on a still runs
+    torch.cuda.synchronize()
+    out = torch.zeros_like(vd)
+    for t in (ta, tb):
+        out.zero_()
+        t.retrieve(kd, out)
+        assert torch.equal(out, vd) and t.size() == n
+
+
 @pytest.mark.parametrize("kb,n,load,shape", [
     (32, 1 << 20, 0.9, "distinct"), (32, 16_000_003, 0.9, "repeats"),   # one pass and two
     (32, 3_000_001, 0.93, "hot"), (32, 16_000_003, 0.9, "few"),

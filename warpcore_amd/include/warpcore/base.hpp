@@ -131,6 +131,16 @@ WC_H unsigned grid_for_lanes(index_t items) noexcept {
     return unsigned(g == 0 ? 1 : g);
 }
 
+// Whether a handle names another stream in every host thread: the per-thread
+// handle, and the null handle where launches on it go to the calling thread's
+// own stream (-fgpu-default-stream=per-thread).
+WC_H bool per_thread_stream(hipStream_t stream) noexcept {
+#if defined(HIP_API_PER_THREAD_DEFAULT_STREAM)
+    if (stream == nullptr) return true;
+#endif
+    return stream == hipStreamPerThread;
+}
+
 // While this object lives, calls of this thread that are not part of a stream
 // capture (allocations, host waits) neither fail nor end a capture that some
 // stream of the process has open in the global or thread-local mode.

@@ -28,16 +28,6 @@
 namespace warpcore {
 namespace detail {
 
-// Whether a handle names another stream in every host thread: the per-thread
-// handle, and the null handle where launches on it go to the calling thread's
-// own stream (-fgpu-default-stream=per-thread).
-WC_H bool per_thread_stream(hipStream_t stream) noexcept {
-#if defined(HIP_API_PER_THREAD_DEFAULT_STREAM)
-    if (stream == nullptr) return true;
-#endif
-    return stream == hipStreamPerThread;
-}
-
 class MutationTracker {
     struct State {
         std::mutex mu;

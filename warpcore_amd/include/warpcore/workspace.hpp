@@ -1,13 +1,13 @@
 // Scratch memory of bulk calls, shared by all tables of the process.
 //
 // A bulk call leases one buffer for the kernels it launches. The lease ends
-// with the call; the buffer is handed out again at once, and its next user's
-// stream first waits (on the device) for the event recorded behind the last
-// user's kernels, so calls on one stream reuse one buffer and calls on
-// several streams or host threads get buffers of their own while the bound
-// allows. Bounded: at most kWorkspaceLimit bytes per device; a lease that
-// would exceed it, or that finds no device memory, is empty and the caller
-// runs its kernels that need no scratch. Given back: the buffers are freed
+// with the call, and an event is recorded behind the call's kernels. A buffer
+// is handed out again to a call on the same stream, or once that event has
+// passed: no stream ever waits for another one's work here, calls on several
+// streams or host threads get buffers of their own. Bounded: at most
+// kWorkspaceLimit bytes per device; a lease that would exceed it, or that
+// finds no device memory, is empty and the caller runs its kernels that need
+// no scratch. Given back: the buffers are freed
 // when the process's last table is destroyed, and idle ones before the bound
 // or the device's memory would refuse a larger lease.
 //
@@ -41,6 +41,7 @@ public:
         std::size_t bytes = 0;
         int device = 0;
         hipEvent_t done = nullptr;   // behind the last user's kernels
+        hipStream_t stream = nullptr;   // the last user's
         bool leased = false;
         Buffer* next = nullptr;
     };
@@ -56,8 +57,8 @@ public:
         free_idle(-1);
     }
 
-    // a buffer of at least `bytes` on the current device, whose earlier use
-    // `stream` waits for; null without one
+    // a buffer of at least `bytes` on the current device whose earlier use is
+    // over or ordered before what `stream` is given next; null without one
     WC_H Buffer* acquire(std::size_t bytes, hipStream_t stream) noexcept {
         bytes = (bytes + kWorkspaceUnit - 1) / kWorkspaceUnit * kWorkspaceUnit;
         int device = 0;
@@ -66,9 +67,11 @@ public:
         const RelaxedCapture relaxed;
         Buffer* best = nullptr;
         for (Buffer* b = first_; b != nullptr; b = b->next)
-            if (!b->leased && b->device == device && b->bytes >= bytes && (best == nullptr || b->bytes < best->bytes))
+            if (!b->leased && b->device == device && b->bytes >= bytes &&
+                (best == nullptr || b->bytes < best->bytes) && (ordered(b, stream) || passed(b)))
                 best = b;
         if (best != nullptr) {
+            // (nothing to wait for unless the handle was given to a new stream)
             if (hipStreamWaitEvent(stream, best->done, 0) != hipSuccess) {
                 (void)hipGetLastError();
                 return nullptr;
@@ -111,6 +114,7 @@ public:
             (void)hipGetLastError();
             (void)hipStreamSynchronize(stream);   // no event to wait for: the kernels end here
         }
+        b->stream = stream;
         b->leased = false;
         if (users_ == 0) free_idle(-1);
     }
@@ -121,6 +125,14 @@ public:
     }
 
 private:
+    WC_H static bool ordered(const Buffer* b, hipStream_t stream) noexcept {
+        return b->stream == stream && !per_thread_stream(stream);
+    }
+    WC_H static bool passed(const Buffer* b) noexcept {
+        const hipError_t e = hipEventQuery(b->done);
+        if (e != hipSuccess && hipPeekAtLastError() == e) (void)hipGetLastError();
+        return e == hipSuccess;
+    }
     // bytes of one device's buffers, or (-1) of all
     WC_H std::size_t held_on(int device) const noexcept {
         std::size_t held = 0;
@@ -128,12 +140,12 @@ private:
             if (device < 0 || b->device == device) held += b->bytes;
         return held;
     }
-    // frees the buffers not leased (of one device, or all); hipFree waits
-    // for the kernels that still use one
+    // frees the buffers not leased: one device's whose last use is over, or
+    // (-1) all, after waiting for the kernels that still use them
     WC_H void free_idle(int device) noexcept {
         for (Buffer** at = &first_; *at != nullptr;) {
             Buffer* b = *at;
-            if (b->leased || (device >= 0 && b->device != device)) {
+            if (b->leased || (device >= 0 && (b->device != device || !passed(b)))) {
                 at = &b->next;
                 continue;
             }
