@@ -210,6 +210,18 @@ WC_API int wc_status_return_any_flag(uint32_t status, uint32_t ignore);
 WC_API int wc_status_to_string(uint32_t status, char* buf, uint64_t len);
 
 /* ------------------------------------------------------------------------
+ * Scratch memory of large bulk inserts (no reference counterpart): buffers
+ * that all tables of the process share, at most 16 GiB per device, kept for
+ * the next insert until the last table is destroyed or a table's own
+ * allocation needs the memory. Not part of any table's _bytes_total.
+ *   _bytes  bytes held on all devices
+ *   _trim   frees the buffers no running call uses, after waiting for the
+ *           kernels that still do; returns the bytes freed
+ * ---------------------------------------------------------------------- */
+WC_API uint64_t wc_workspace_bytes(void);
+WC_API uint64_t wc_workspace_trim(void);
+
+/* ------------------------------------------------------------------------
  * CountingHashTable<K, uint64_t> (include/warpcore/counting_hash_table.cuh)
  *   _create (min_capacity, seed, max_count, no_init)               :74-85
  *   _init / _init_seed                                              :113-135

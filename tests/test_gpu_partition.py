@@ -188,6 +188,58 @@ def test_insert_beside_a_capture_of_another_stream(cuda):
         assert bool((x == 3 * (replay + 1)).all())
 
 
+def test_workspace_is_given_back(cuda):
+    """Kept between inserts and reused, given back by a trim, by the last
+    table's end, and where a table's own allocation needs the memory; refused
+    where it would take more than half of what is free."""
+    import gc
+    from warpcore_amd.tables import HashSet, SingleValueHashTable, trim_workspace, workspace_bytes
+    gc.collect()
+    trim_workspace()
+    assert workspace_bytes() == 0
+    n = 20_000_003
+    keys = unique_keys(n, 64, seed=27)
+    kd = to_dev(keys)
+    t = SingleValueHashTable(math.ceil(n / 0.85), 64, 64)
+    small = SingleValueHashTable(1 << 22, 64, 64)
+    small.insert(kd[:3_000_000], kd[:3_000_000])
+    first = workspace_bytes()
+    assert 0 < first < 1 << 30
+    t.insert(kd, kd)
+    held = workspace_bytes()
+    assert held > first
+    small.init()
+    small.insert(kd[:3_000_000], kd[:3_000_000])
+    t.init()
+    t.insert(kd, kd)
+    assert workspace_bytes() == held
+    # a card as good as full: the next table gets the workspace's memory
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    want = (held - first) // 2
+    hog = []
+    while len(hog) < 8 and torch.cuda.mem_get_info()[0] >= want:
+        hog.append(torch.empty(torch.cuda.mem_get_info()[0] - want // 2, dtype=torch.uint8, device="cuda"))
+    assert torch.cuda.mem_get_info()[0] < want
+    late = HashSet(want // 8, 64)
+    assert int(late.peek_status()) == S_NONE and workspace_bytes() == 0
+    # too little left for a workspace: the insert runs without
+    out = torch.zeros_like(kd[:1 << 20])
+    small.init()
+    small.insert(kd[:3_000_000], kd[:3_000_000])
+    small.retrieve(kd[:1 << 20], out)
+    assert small.size() == 3_000_000 and torch.equal(out, kd[:1 << 20])
+    del hog, late
+    torch.cuda.empty_cache()
+    small.init()
+    small.insert(kd[:3_000_000], kd[:3_000_000])
+    assert workspace_bytes() == first and trim_workspace() == first and workspace_bytes() == 0
+    t.init()
+    t.insert(kd, kd)
+    t.retrieve(kd[:1 << 20], out)
+    assert t.size() == n and torch.equal(out, kd[:1 << 20])
+
+
 def _streams_side_by_side():
     """Two streams whose kernels do run beside each other (streams share a few
     hardware queues)."""

@@ -295,7 +295,7 @@ public:
         : bloom_filter_(nullptr), num_bits_(num_bits), num_slots_(SDIV(num_bits, slot_bits())),
           num_blocks_(SDIV(num_slots_, cg_size())), mod_blocks_(num_blocks_ ? num_blocks_ : 1),
           mod_slots_(num_slots_ ? num_slots_ : 1), k_(k), seed_(seed), is_copy_(false) {
-        if (num_slots_ != 0 && hipMalloc(&bloom_filter_, sizeof(slot_type) * num_slots_) != hipSuccess)
+        if (num_slots_ != 0 && detail::device_malloc(&bloom_filter_, sizeof(slot_type) * num_slots_) != hipSuccess)
             bloom_filter_ = nullptr;
         detail::WorkspacePool::instance().add_user();
         init();

@@ -561,9 +561,9 @@ public:
         if (capacity_ < handle_type::max_bucket_index() && bucket_grow_factor_ >= 1.0f && min_bucket_size_ >= 1 &&
             max_bucket_size_ >= min_bucket_size_ && max_bucket_size_ <= handle_type::max_bucket_size()) {
             const std::size_t bytes = sizeof(bucket_type) * capacity_ + counter_bytes();
-            if (warpcore::detail::available_gpu_memory() >= bytes &&
-                (capacity_ == 0 || hipMalloc(&buckets_, sizeof(bucket_type) * capacity_) == hipSuccess) &&
-                hipMalloc(&counters_, counter_bytes()) == hipSuccess) {
+            if (warpcore::detail::device_memory_for(bytes) &&
+                (capacity_ == 0 || warpcore::detail::device_malloc(&buckets_, sizeof(bucket_type) * capacity_) == hipSuccess) &&
+                warpcore::detail::device_malloc(&counters_, counter_bytes()) == hipSuccess) {
                 status_ = Status::none();
                 init();
             } else {
@@ -1181,7 +1181,7 @@ public:
           value_store_(value_capacity, grow_factor, min_bucket_size, max_bucket_size_),
           max_values_per_key_(std::min(max_values_per_key, handle_type::max_value_count())), is_copy_(false),
           scan_parts_(nullptr) {
-        if (hipMalloc(&scan_parts_, sizeof(index_type) * warpcore::detail::kScanParts) != hipSuccess) {
+        if (warpcore::detail::device_malloc(&scan_parts_, sizeof(index_type) * warpcore::detail::kScanParts) != hipSuccess) {
             scan_parts_ = nullptr;
             join_status(Status::out_of_memory());
         }
@@ -1548,7 +1548,7 @@ private:
         if (scratch_ != nullptr) (void)hipFree(scratch_);
         scratch_ = nullptr;
         scratch_cap_ = 0;
-        if (hipMalloc(&scratch_, 2 * sizeof(std::uint32_t) * n) != hipSuccess) {
+        if (warpcore::detail::device_malloc(&scratch_, 2 * sizeof(std::uint32_t) * n) != hipSuccess) {
             scratch_ = nullptr;
             return false;
         }

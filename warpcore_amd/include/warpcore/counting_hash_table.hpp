@@ -843,7 +843,7 @@ private:
         WC_H bool reserve(index_type n) noexcept {
             if (n <= capacity) return true;
             release();
-            if (hipMalloc(&base, CombineBuffers::bytes_for(n)) != hipSuccess) {
+            if (detail::device_malloc(&base, CombineBuffers::bytes_for(n)) != hipSuccess) {
                 base = nullptr;
                 return false;
             }

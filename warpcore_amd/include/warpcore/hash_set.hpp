@@ -168,9 +168,9 @@ public:
           geo_(probing_schemes::Geometry::make(capacity_, cg_size())) {
         detail::WorkspacePool::instance().add_user();
         const std::size_t bytes = sizeof(key_type) * capacity_;
-        if (hipMalloc(&status_, sizeof(status_type)) != hipSuccess) { status_ = nullptr; return; }
+        if (detail::device_malloc(&status_, sizeof(status_type)) != hipSuccess) { status_ = nullptr; return; }
         if (capacity_ == 0) { assign_status(Status::invalid_configuration() + Status::not_initialized()); return; }
-        if (detail::available_gpu_memory() < bytes || hipMalloc(&keys_, bytes) != hipSuccess) {
+        if (!detail::device_memory_for(bytes) || detail::device_malloc(&keys_, bytes) != hipSuccess) {
             keys_ = nullptr;
             assign_status(Status::out_of_memory() + Status::not_initialized());
             return;

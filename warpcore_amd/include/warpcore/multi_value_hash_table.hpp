@@ -439,9 +439,9 @@ public:
           temp_(TempMemoryBytes / sizeof(index_type)), seed_(seed), max_values_per_key_(max_values_per_key),
           num_keys_(nullptr), scan_parts_(nullptr), is_copy_(false), is_initialized_(false),
           geo_(probing_schemes::Geometry::make(table_.capacity(), cg_size())) {
-        if (hipMalloc(&status_, sizeof(status_type)) != hipSuccess) status_ = nullptr;
-        if (hipMalloc(&num_keys_, sizeof(index_type)) != hipSuccess) num_keys_ = nullptr;
-        if (hipMalloc(&scan_parts_, sizeof(index_type) * detail::kScanParts) != hipSuccess) scan_parts_ = nullptr;
+        if (detail::device_malloc(&status_, sizeof(status_type)) != hipSuccess) status_ = nullptr;
+        if (detail::device_malloc(&num_keys_, sizeof(index_type)) != hipSuccess) num_keys_ = nullptr;
+        if (detail::device_malloc(&scan_parts_, sizeof(index_type) * detail::kScanParts) != hipSuccess) scan_parts_ = nullptr;
         status_type st = table_.status() + temp_.status();
         if (num_keys_ == nullptr || scan_parts_ == nullptr) st += Status::out_of_memory() + Status::not_initialized();
         assign_status(st);

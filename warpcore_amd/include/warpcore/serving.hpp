@@ -398,7 +398,7 @@ private:
     template<class T>
     static bool alloc(T** p, index_t n) {
         *p = nullptr;
-        return hipMalloc(reinterpret_cast<void**>(p), sizeof(T) * (n ? n : 1)) == hipSuccess;
+        return warpcore::detail::device_malloc(p, sizeof(T) * (n ? n : 1)) == hipSuccess;
     }
 
     // under mu_

@@ -467,9 +467,9 @@ public:
           is_initialized_(false),
           is_copy_(false),
           geo_(probing_schemes::Geometry::make(table_.capacity(), cg_size())) {
-        if (hipMalloc(&status_, sizeof(status_type)) != hipSuccess) status_ = nullptr;
+        if (detail::device_malloc(&status_, sizeof(status_type)) != hipSuccess) status_ = nullptr;
         if constexpr (with_filter) {
-            if (table_.capacity() != 0 && hipMalloc(&filter_, filter_bytes()) != hipSuccess) filter_ = nullptr;
+            if (table_.capacity() != 0 && detail::device_malloc(&filter_, filter_bytes()) != hipSuccess) filter_ = nullptr;
         }
         assign_status(table_.status() + temp_.status());
         detail::WorkspacePool::instance().add_user();

@@ -15,6 +15,7 @@
 #include "base.hpp"
 #include "status.hpp"
 #include "tags.hpp"
+#include "workspace.hpp"
 
 #include <atomic>
 
@@ -41,8 +42,8 @@ public:
     WC_H explicit CyclicStore(index_type capacity) noexcept
         : store_(nullptr), capacity_(capacity), current_(nullptr), status_(Status::not_initialized()), is_copy_(false) {
         if (capacity_ == 0) { status_ += Status::invalid_configuration(); return; }
-        if (warpcore::detail::available_gpu_memory() < sizeof(T) * capacity_ ||
-            hipMalloc(&store_, sizeof(T) * capacity_) != hipSuccess) {
+        if (!warpcore::detail::device_memory_for(sizeof(T) * capacity_) ||
+            warpcore::detail::device_malloc(&store_, sizeof(T) * capacity_) != hipSuccess) {
             store_ = nullptr;
             status_ += Status::out_of_memory();
             return;
@@ -114,8 +115,8 @@ public:
         : status_(Status::not_initialized()), capacity_(capacity), keys_(nullptr), values_(nullptr), is_copy_(false) {
         if (capacity_ == 0) { status_ += Status::invalid_configuration(); return; }
         const std::size_t bytes = (sizeof(Key) + sizeof(Value)) * capacity_;
-        if (warpcore::detail::available_gpu_memory() < bytes || hipMalloc(&keys_, sizeof(Key) * capacity_) != hipSuccess ||
-            hipMalloc(&values_, sizeof(Value) * capacity_) != hipSuccess) {
+        if (!warpcore::detail::device_memory_for(bytes) || warpcore::detail::device_malloc(&keys_, sizeof(Key) * capacity_) != hipSuccess ||
+            warpcore::detail::device_malloc(&values_, sizeof(Value) * capacity_) != hipSuccess) {
             release();
             status_ += Status::out_of_memory();
             return;
@@ -182,7 +183,7 @@ public:
         : status_(Status::not_initialized()), capacity_(capacity), pairs_(nullptr), is_copy_(false) {
         if (capacity_ == 0) { status_ += Status::invalid_configuration(); return; }
         const std::size_t bytes = sizeof(slot_type) * capacity_;
-        if (warpcore::detail::available_gpu_memory() < bytes || hipMalloc(&pairs_, bytes) != hipSuccess) {
+        if (!warpcore::detail::device_memory_for(bytes) || warpcore::detail::device_malloc(&pairs_, bytes) != hipSuccess) {
             pairs_ = nullptr;
             status_ += Status::out_of_memory();
             return;

@@ -608,7 +608,7 @@ private:
     template<class T>
     WC_H static bool malloc_(T** p, std::size_t bytes) noexcept {
         *p = nullptr;
-        return hipMalloc(reinterpret_cast<void**>(p), bytes ? bytes : 1) == hipSuccess;
+        return warpcore::detail::device_malloc(p, bytes ? bytes : 1) == hipSuccess;
     }
 
     template<class StatusHandler, bool IsInsert>

@@ -7,9 +7,11 @@
 // streams or host threads get buffers of their own. Bounded: at most
 // kWorkspaceLimit bytes per device; a lease that would exceed it, or that
 // finds no device memory, is empty and the caller runs its kernels that need
-// no scratch. Given back: the buffers are freed
-// when the process's last table is destroyed, and idle ones before the bound
-// or the device's memory would refuse a larger lease.
+// no scratch; so does one that would leave less device memory free than it
+// takes. Given back: the buffers are freed when the process's last table is
+// destroyed, by trim(), where a table's own allocation finds too little memory
+// (device_malloc, device_memory_for), and before the bound or the device's
+// memory would refuse a larger lease.
 //
 // Not for calls under stream capture: a graph would keep the buffer's address
 // beyond the lease. Beside a capture of another stream the pool allocates and
@@ -92,15 +94,12 @@ public:
             delete b;
             return nullptr;
         }
-        if (hipMalloc(&b->p, bytes) != hipSuccess) {
+        if (available_gpu_memory() / 2 < bytes) free_idle(device);
+        if (available_gpu_memory() / 2 < bytes || hipMalloc(&b->p, bytes) != hipSuccess) {
             (void)hipGetLastError();
-            free_idle(device);
-            if (hipMalloc(&b->p, bytes) != hipSuccess) {
-                (void)hipGetLastError();
-                (void)hipEventDestroy(b->done);
-                delete b;
-                return nullptr;
-            }
+            (void)hipEventDestroy(b->done);
+            delete b;
+            return nullptr;
         }
         b->leased = true;
         b->next = first_;
@@ -117,6 +116,15 @@ public:
         b->stream = stream;
         b->leased = false;
         if (users_ == 0) free_idle(-1);
+    }
+    // frees the buffers no call holds, after waiting for the kernels that
+    // still use them; the bytes freed, on all devices
+    WC_H std::size_t trim() noexcept {
+        std::lock_guard<std::mutex> lock(mu_);
+        const RelaxedCapture relaxed;
+        const std::size_t before = held_on(-1);
+        free_idle(-1);
+        return before - held_on(-1);
     }
     // bytes held on all devices
     WC_H std::size_t bytes_held() noexcept {
@@ -161,6 +169,20 @@ private:
     Buffer* first_ = nullptr;   // linked in the buffers themselves: a lease allocates nothing that may throw
     std::size_t users_ = 0;
 };
+
+// Allocations of the tables themselves, before which idle scratch memory goes
+// back: whether the device has `bytes` free, and hipMalloc.
+WC_H bool device_memory_for(std::size_t bytes) noexcept {
+    return available_gpu_memory() >= bytes ||
+           (WorkspacePool::instance().trim() != 0 && available_gpu_memory() >= bytes);
+}
+template<class T>
+WC_H hipError_t device_malloc(T** p, std::size_t bytes) noexcept {
+    const hipError_t e = hipMalloc(reinterpret_cast<void**>(p), bytes);
+    if (e == hipSuccess || WorkspacePool::instance().trim() == 0) return e;
+    (void)hipGetLastError();
+    return hipMalloc(reinterpret_cast<void**>(p), bytes);
+}
 
 // One bulk call's lease; false when the pool has no buffer for it.
 class WorkspaceLease {

@@ -876,6 +876,18 @@ class Server:
         return lat, mk.value
 
 
+def workspace_bytes() -> int:
+    """Device memory that large bulk inserts keep as scratch (no table's
+    bytes_total includes it)."""
+    return _capi.lib().wc_workspace_bytes()
+
+
+def trim_workspace() -> int:
+    """Frees that memory, after the kernels that still use it; returns the
+    bytes freed. It comes back with the next large insert."""
+    return _capi.lib().wc_workspace_trim()
+
+
 def load_binary(path, key_bits: int = 64, max_keys: int = 1 << 27):
     """Keys of a raw little-endian key file (the reference benchmarks'
     load_keys input format, benchmarks/include/benchmark_common.cuh:62-75),
