@@ -19,6 +19,9 @@ int wcp_per_thread_stream(int which) {
     return detail::per_thread_stream(s[which]) ? 1 : 0;
 }
 
+// grid of the region passes' launches (no device call)
+unsigned wcp_part_blocks(std::uint64_t wanted, unsigned resident) { return detail::part_blocks(wanted, resident); }
+
 // `parts` equal shares of the keys, each inserted by a host thread of its own,
 // one call after another, none waited for; returns the keys stored. The
 // values are the keys.

@@ -855,8 +855,14 @@ constexpr bool partition_capable() noexcept {
            status_handlers::overwrites<StatusHandler>::value;
 }
 
-// Grid of a launch whose blocks are dealt to the XCDs in turn: a multiple of
-// 8, at most the resident blocks.
+// Grid of a launch whose blocks are dealt to the XCDs in turn: a multiple of 8
+// (part_refine strides by eighths of it), at most the resident blocks where
+// there are as many.
+constexpr unsigned part_blocks(index_t wanted, unsigned resident) noexcept {
+    const index_t up = SDIV(wanted < 1 ? 1 : wanted, index_t(kPartXcds)) * kPartXcds;
+    const unsigned most = resident < kPartXcds ? kPartXcds : resident / kPartXcds * kPartXcds;
+    return unsigned(up < most ? up : most);
+}
 template<auto Kernel>
 WC_H unsigned part_grid(index_t wanted) noexcept {
     static const unsigned resident = [] {
@@ -866,8 +872,7 @@ WC_H unsigned part_grid(index_t wanted) noexcept {
             blocks = 1;
         return unsigned(num_compute_units()) * unsigned(blocks);
     }();
-    const index_t up = SDIV(wanted < 1 ? 1 : wanted, index_t(kPartXcds)) * kPartXcds;
-    return unsigned(up < resident ? up : resident);
+    return part_blocks(wanted, resident);
 }
 
 // Whether a batch of n keys is partitioned. Below 2^20 keys the passes'
