@@ -99,9 +99,32 @@ std::int64_t lists(const K* keys, index_t n, index_t key_capacity, unsigned copi
     return std::int64_t(bad);
 }
 
+// Pairs stored by one call with buckets of 2^26 + 2^14 values in a pool of
+// 2^27 - 2 cells, none of whose arenas holds one: the values are the keys' positions.
+// The table's status word goes to *status.
+std::int64_t large_buckets(const std::uint32_t* keys, index_t n, bool statuses, std::uint32_t* status) {
+    using store = storage::multi_value::BucketListStore<std::uint32_t, 27, 8, 27>;
+    BucketListHashTable<std::uint32_t, std::uint32_t, defaults::empty_key<std::uint32_t>(),
+                        defaults::tombstone_key<std::uint32_t>(), store>
+        table(n / 2, (index_t(1) << 27) - 2, defaults::seed<std::uint32_t>(), 1.1f, (1u << 26) + (1u << 14));
+    Buffer<Status> out(n);
+    if (out.p == nullptr) return -1;
+    if (statuses)
+        table.insert<status_handlers::ReturnStatus>(keys, keys, n, 0, defaults::probing_length(), out.p);
+    else
+        table.insert(keys, keys, n);
+    *status = table.peek_status().base();
+    const std::int64_t stored = std::int64_t(table.num_values());
+    return hipDeviceSynchronize() == hipSuccess ? stored : -1;
+}
+
 }  // namespace
 
 extern "C" {
+
+std::int64_t wcv_large_buckets(const std::uint32_t* keys, std::uint64_t n, int statuses, std::uint32_t* status) {
+    return large_buckets(keys, n, statuses != 0, status);
+}
 
 // kind 0 <u64, 32 bytes>, 1 <u64, 16 bytes>, 2 <u32, 12 bytes>; lists: 3 <u32, defaulted>
 std::int64_t wcv_single(int kind, const void* keys, std::uint64_t n, std::uint64_t min_capacity) {

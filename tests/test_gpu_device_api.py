@@ -256,3 +256,17 @@ def test_insert_without_host_memory(cuda):
     torch.cuda.synchronize()
     assert lib.wch_insert(_p(kd), n, int(n / 0.9), _p(out)) == n
     assert torch.equal(out, kd)
+
+
+@pytest.mark.parametrize("statuses", [0, 1])
+def test_lists_with_buckets_larger_than_an_arena(vlib, statuses):
+    """Grouped and pair by pair: buckets whose 64-fold size does not fit 32
+    bits and of which the pool holds none. Every key is stored, no value is."""
+    vlib.wcv_large_buckets.restype = ctypes.c_int64
+    vlib.wcv_large_buckets.argtypes = [ctypes.c_void_p, ctypes.c_uint64, ctypes.c_int, ctypes.c_void_p]
+    n = 1_300_000   # more pairs than slots
+    kd = to_dev(np.tile(unique_keys(20_000, 32, seed=81), n // 20_000))
+    word = ctypes.c_uint32(0)
+    torch.cuda.synchronize()
+    assert vlib.wcv_large_buckets(_p(kd), n, statuses, ctypes.byref(word)) == 0
+    assert word.value == S_DUP | 1 << 7   # duplicate_key, out_of_memory

@@ -334,13 +334,13 @@ struct BucketListStoreView {
             if (room == 0) {
                 const bool headed = h.count != 0;
                 const small_type larger = headed ? grown(h.size) : first;
-                const std::uint32_t need = std::uint32_t(larger) + (headed ? 1 : 0);
+                const index_t need = index_t(larger) + (headed ? 1 : 0);
                 index_t alloc = run;
                 if (need <= cells) {
                     run += need;
-                    cells -= need;
+                    cells -= std::uint32_t(need);
                 } else {
-                    alloc = allocate(index_t(larger) + (headed ? 1 : 0));
+                    alloc = allocate(need);
                 }
                 if (alloc == ~index_t(0)) {
                     st = Status::out_of_memory();
@@ -396,8 +396,11 @@ struct BucketListStoreView {
     // try have the cells of all their buckets allocated by one atomic, where
     // the wavefront's arena holds them (2^26 pairs over 2^23 keys: the groups
     // pass 3.65 ms, bucket by bucket, an atomic's round trip each, 4.07); the
-    // others append on their own after those have published.
+    // others append on their own after those have published. A lane that would
+    // take kMostCells cells or more takes them bucket by bucket, so that a
+    // wavefront's sum fits 32 bits for any bucket sizes.
     // (`fresh`: the handle of a key just claimed, taken to be uninitialised.)
+    static constexpr std::uint32_t kMostCells = 1u << 20;
     template<class Next>
     WC_D Status append_wave(bool on, bool fresh, handle_type* handle, small_type pairs, const Next& next,
                             index_t max_values_per_key) const noexcept {
@@ -419,12 +422,13 @@ struct BucketListStoreView {
             small_type size = h.size, room = headed ? size - h.tail : 0;
             const small_type most = small_type(max_values_per_key) - h.count;
             small_type more = most < pairs ? most : pairs;
-            while (more > room && cells < (1u << 20)) {
+            while (more > room && cells < kMostCells) {
                 more -= room;
                 room = size = headed ? grown(size) : small_type(min_size);
-                cells += std::uint32_t(size) + (headed ? 1 : 0);
+                cells = size < kMostCells ? cells + std::uint32_t(size) + (headed ? 1 : 0) : kMostCells;
                 headed = true;
             }
+            if (cells >= kMostCells) cells = 0;
         }
         std::uint32_t upto = cells;
 #pragma unroll
