@@ -500,3 +500,23 @@ def test_pairs_insert_limits(cuda):
     assert n // 8 < total <= n // 2
     owner, v = _values_by_key(small, uniq, 32, total)
     assert len(np.unique(v)) == total and (uniq[owner] == keys[v.astype(np.int64) - 1]).all()
+
+
+@pytest.mark.parametrize("distinct", [1 << 18, 1 << 20])
+def test_pairs_insert_tight_pool(cuda, distinct):
+    """Eight values per key in buckets of 1, 2, 3 and 4 (13 cells) and a pool
+    of just so many cells and, per arena, the 4 that a bucket of 5 cells may
+    leave: everything is stored."""
+    from warpcore_amd.tables import BucketListHashTable
+    n = 8 * distinct
+    keys = np.tile(unique_keys(distinct, 32, seed=distinct), 8)
+    np.random.default_rng(3).shuffle(keys)
+    kd, vd = to_dev(keys), torch.arange(n, dtype=torch.int32, device="cuda")
+    arenas = 1
+    while arenas < 256 and 13 * distinct // (2 * arenas) >= 1 << 16:
+        arenas *= 2
+    t = BucketListHashTable(math.ceil(distinct / 0.9), 13 * distinct + 4 * arenas, 32, 32, grow_factor=1.1,
+                            min_bucket_size=1)
+    t.insert(kd, vd)
+    assert int(t.pop_status()) == S_DUP
+    assert t.num_keys() == distinct and t.num_values() == n

@@ -400,7 +400,7 @@ struct BucketListStoreView {
     // take kMostCells cells or more takes them bucket by bucket, so that a
     // wavefront's sum fits 32 bits for any bucket sizes.
     // (`fresh`: the handle of a key just claimed, taken to be uninitialised.)
-    static constexpr std::uint32_t kMostCells = 1u << 20;
+    static constexpr std::uint32_t kMostCells = 1u << 20, kWaveCells = 4096;
     template<class Next>
     WC_D Status append_wave(bool on, bool fresh, handle_type* handle, small_type pairs, const Next& next,
                             index_t max_values_per_key) const noexcept {
@@ -441,10 +441,27 @@ struct BucketListStoreView {
         if (total != 0) {   // uniform
             const index_t a = home_arena();
             if (warpcore::lane_id() == 0) {
+                // A request that does not fit leaves the arena's last cells to
+                // smaller ones, so near the end it is a compare-and-swap (an
+                // add would move the counter past them; the counter only
+                // grows, so the loop ends). Further off an add is safe: each
+                // wavefront of this arena has one at most under way, of
+                // kWaveCells at most (2^26 pairs over 2^23 keys: 5.51 ms, with
+                // the swap alone 5.61).
                 index_t* counter = counters + a * kCounterStride;
-                if (warpcore::detail::atomic_load_relaxed(counter) + total <= arena_size(a)) {
-                    const index_t at = warpcore::detail::atomic_add(counter, index_t(total));
-                    if (at + total <= arena_size(a)) run = arena_begin(a) + at;
+                const index_t waves = SDIV(index_t(gridDim.x) * (blockDim.x >> 6), arenas);
+                index_t at = warpcore::detail::atomic_load_relaxed(counter);
+                if (total <= kWaveCells && at + waves * kWaveCells <= arena_size(a)) {
+                    run = arena_begin(a) + warpcore::detail::atomic_add(counter, index_t(total));
+                    at = arena_size(a);
+                }
+                while (at + total <= arena_size(a)) {
+                    const index_t seen = warpcore::detail::atomic_cas(counter, at, at + total);
+                    if (seen == at) {
+                        run = arena_begin(a) + at;
+                        break;
+                    }
+                    at = seen;
                 }
             }
             run = (index_t(unsigned(__builtin_amdgcn_readfirstlane(int(run >> 32)))) << 32) |
