@@ -247,6 +247,24 @@ int store_check(std::uint64_t capacity, unsigned long long* errors) {
 
 
 
+template<unsigned CG>
+void group_plan(index_t n, index_t capacity, std::uint64_t* out) {
+    using K = std::uint32_t;
+    using store = storage::multi_value::BucketListStore<K>;
+    using view = typename SingleValueHashTable<K, store::handle_type, defaults::empty_key<K>(),
+                                               defaults::tombstone_key<K>(),
+                                               defaults::probing_scheme_t<K, CG>>::view_type;
+    using core = detail::BucketListGroupCore<view, store::view_type>;
+    using record = detail::PairRecord<K, K>;
+    const auto geo = probing_schemes::Geometry::make(capacity, CG);
+    const auto p = detail::make_part_plan<detail::PairSortCore<view, K>, record, false>(
+        n, geo, detail::group_windows<core, record>(n, geo), detail::kGroupSigmas);
+    out[0] = p.cap1;
+    out[1] = p.two_pass() ? p.cap2 : 0;
+    out[2] = p.buckets;
+    out[3] = p.two_pass();
+}
+
 }  // namespace
 
 extern "C" {
@@ -391,6 +409,27 @@ int wcx_handler_calls(int which, const std::uint64_t* keys, std::uint64_t n, std
     HashSet<std::uint64_t> set(capacity);
     set.insert<CountCalls>(keys, n, 0, defaults::probing_length(), calls_out);
     return int(hipDeviceSynchronize());
+}
+
+// The host's bulk insert into the table of wcx_svht_create; scratch memory that
+// this library's bulk inserts keep, and freeing it.
+void wcx_svht_insert(void* t, const std::uint64_t* keys, const std::uint64_t* values, std::uint64_t n, void* stream) {
+    static_cast<SingleValueHashTable<std::uint64_t, std::uint64_t>*>(t)->insert(keys, values, n,
+                                                                             static_cast<hipStream_t>(stream));
+}
+void wcx_svht_init(void* t, void* stream) {
+    static_cast<SingleValueHashTable<std::uint64_t, std::uint64_t>*>(t)->init(static_cast<hipStream_t>(stream));
+}
+std::uint64_t wcx_workspace_bytes() { return detail::WorkspacePool::instance().bytes_held(); }
+std::uint64_t wcx_workspace_trim() { return detail::WorkspacePool::instance().trim(); }
+
+// Segment sizes of a grouped insert of n pairs of u32 into a
+// BucketListHashTable of cg 4 or 8 and `capacity` slots (no device call):
+// records per (bucket, XCD) and per region, buckets, and whether there are
+// two passes.
+void wcx_group_plan(unsigned cg, std::uint64_t n, std::uint64_t capacity, std::uint64_t* out) {
+    if (cg == 4) group_plan<4>(n, capacity, out);
+    else group_plan<8>(n, capacity, out);
 }
 
 }  // extern "C"

@@ -270,3 +270,38 @@ def test_lists_with_buckets_larger_than_an_arena(vlib, statuses):
     torch.cuda.synchronize()
     assert vlib.wcv_large_buckets(_p(kd), n, statuses, ctypes.byref(word)) == 0
     assert word.value == S_DUP | 1 << 7   # duplicate_key, out_of_memory
+
+
+def test_bulk_inserts_beside_a_copy_of_the_table(dlib):
+    """A copy handed to a kernel waits for the region insert that still runs,
+    and from then on, init() included, bulk inserts run beside anything."""
+    P, U64 = ctypes.c_void_p, ctypes.c_uint64
+    dlib.wcx_svht_insert.restype = dlib.wcx_svht_init.restype = None
+    dlib.wcx_svht_insert.argtypes = [P, P, P, U64, P]
+    dlib.wcx_svht_init.argtypes = [P, P]
+    dlib.wcx_workspace_bytes.restype = dlib.wcx_workspace_trim.restype = U64
+    n, m = 2_000_000, 200_000
+    keys = unique_keys(2 * n + m, 64, seed=91)
+    kd = to_dev(keys)
+    out, st = torch.zeros_like(kd), torch.zeros(len(keys), dtype=torch.int32, device="cuda")
+    s = torch.cuda.Stream()   # does not order itself against the null stream, on which the kernels below run
+    h = dlib.wcx_svht_create(int(len(keys) / 0.9))
+    try:
+        torch.cuda.synchronize()
+        dlib.wcx_workspace_trim()
+        for round_ in range(2):
+            dlib.wcx_svht_insert(h, _p(kd), _p(kd), n, P(s.cuda_stream))
+            assert (dlib.wcx_workspace_bytes() > 0) == (round_ == 0)
+            assert dlib.wcx_svht_phase(h, 0, _p(kd[2 * n:]), _p(kd[2 * n:]), m, None, _p(st)) == 0
+            dlib.wcx_workspace_trim()
+            dlib.wcx_svht_insert(h, _p(kd[n:]), _p(kd[n:]), n, P(s.cuda_stream))
+            assert dlib.wcx_workspace_bytes() == 0
+            torch.cuda.synchronize()
+            out.zero_()
+            torch.cuda.synchronize()
+            assert dlib.wcx_svht_phase(h, 1, _p(kd), None, len(keys), _p(out), _p(st)) == 0
+            assert torch.equal(out, kd) and int(st.abs().sum()) == 0
+            dlib.wcx_svht_init(h, P(s.cuda_stream))
+            torch.cuda.synchronize()
+    finally:
+        dlib.wcx_svht_destroy(h)

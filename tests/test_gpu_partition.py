@@ -137,33 +137,56 @@ def test_insert_on_stored_keys(cuda, kb, vb, cg):
     np.testing.assert_array_equal(from_dev(out, dtype(vb)), _value_of(keys, vb))
 
 
+def _sorted(insert):
+    """Whether insert() sorts its batch by region: what it leaves in the
+    library's workspace after a trim."""
+    from warpcore_amd.tables import trim_workspace, workspace_bytes
+    trim_workspace()
+    insert()
+    return workspace_bytes() > 0
+
+
 def test_inserts_from_two_streams(cuda):
-    """Batches inserted on two streams without synchronization: every key is
-    stored, whichever batch was partitioned."""
+    """Batches large enough for the region passes on two streams, without
+    synchronization: the first one on `a` is sorted, the one on `b` waits for
+    it and takes the general kernels, as everything does until init()."""
     from warpcore_amd.tables import SingleValueHashTable
-    n = 2_000_000
-    keys = unique_keys(3 * n, 64, seed=21)
+    n = 2_000_000   # 0.41 of the slots
+    keys = unique_keys(2 * n, 64, seed=21)
     vals = _value_of(keys, 64)
     kd, vd = to_dev(keys), to_dev(vals)
     a, b = torch.cuda.Stream(), torch.cuda.Stream()
-    t = SingleValueHashTable(math.ceil(3 * n / 0.85), 64, 64)
+    t = SingleValueHashTable(math.ceil(2 * n / 0.9), 64, 64)
+    assert t.capacity() * 3 // 8 < n
+
+    def part(i, s):
+        t.insert(kd[i * n:(i + 1) * n], vd[i * n:(i + 1) * n], stream=s)
+
     torch.cuda.synchronize()
-    for round_ in range(3):   # the first round's insert on `a` is partitioned, the one on `b` waits for it
+    for round_ in range(3):
         t.init(stream=a)
-        for i, s in enumerate((a, b, a)):
-            t.insert(kd[i * n:(i + 1) * n], vd[i * n:(i + 1) * n], stream=s)
+        part(0, a)
+        part(1, b)
         torch.cuda.synchronize()
-        assert t.size() == 3 * n
+        assert t.size() == 2 * n
         out = torch.zeros_like(vd)
         t.retrieve(kd, out, stream=a)
         torch.cuda.synchronize()
         assert torch.equal(out, vd)
+    t.init(stream=a)
+    assert _sorted(lambda: part(0, a))
+    assert not _sorted(lambda: part(1, b))
+    assert not _sorted(lambda: part(0, a))   # the table has seen two streams
+    t.init(stream=a)
+    assert _sorted(lambda: part(0, a)) and _sorted(lambda: part(1, a))
+    torch.cuda.synchronize()
+    assert t.size() == 2 * n
 
 
 def test_insert_beside_a_capture_of_another_stream(cuda):
     """A bulk insert whose workspace is allocated while another stream is
     captured in the global mode: the insert runs, the capture stays valid."""
-    from warpcore_amd.tables import BloomFilter, SingleValueHashTable
+    from warpcore_amd.tables import BloomFilter, SingleValueHashTable, trim_workspace
     n = 3_000_001
     keys = unique_keys(n, 64, seed=23)
     kd, vd = to_dev(keys), to_dev(_value_of(keys, 64))
@@ -171,6 +194,7 @@ def test_insert_beside_a_capture_of_another_stream(cuda):
     x = torch.zeros(1024, device="cuda")
     a, b = torch.cuda.Stream(), torch.cuda.Stream()
     g = torch.cuda.CUDAGraph()
+    trim_workspace()
     torch.cuda.synchronize()
     with torch.cuda.graph(g, stream=b, capture_error_mode="global"):
         x.add_(1)
@@ -238,6 +262,85 @@ def test_workspace_is_given_back(cuda):
     t.insert(kd, kd)
     t.retrieve(kd[:1 << 20], out)
     assert t.size() == n and torch.equal(out, kd[:1 << 20])
+
+
+def test_other_inserts_without_a_workspace(cuda, oracle):
+    """Sets, counters, filters and bucket lists where too little memory is free
+    for a workspace: the general kernels."""
+    from warpcore_amd.tables import (BloomFilter, BucketListHashTable, CountingHashTable, HashSet, trim_workspace,
+                                     workspace_bytes)
+    n = 5_000_001
+    keys = unique_keys(n, 64, seed=29)
+    kd = to_dev(keys)
+    h, c = HashSet(math.ceil(n / 0.9), 64), CountingHashTable(math.ceil(n / 0.9), 64)
+    bf, bl = BloomFilter(1 << 27, 4, 64), BucketListHashTable(math.ceil(n / 2 / 0.9), 2 * n, 64, 64)
+    six = kd[: n // 6].repeat(6)
+    flags, counts = torch.zeros(n, dtype=torch.uint8, device="cuda"), torch.zeros(n, dtype=torch.int64, device="cuda")
+    c.insert(kd)   # its own combining buffers
+    c.init()
+    trim_workspace()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    hog = []
+    while len(hog) < 8 and torch.cuda.mem_get_info()[0] >= 64 << 20:
+        hog.append(torch.empty(torch.cuda.mem_get_info()[0] - (40 << 20), dtype=torch.uint8, device="cuda"))
+    free = torch.cuda.mem_get_info()[0]
+    h.insert(kd)
+    c.insert(kd)
+    bf.insert(kd)
+    bl.insert(six, six)
+    held = workspace_bytes()
+    del hog
+    torch.cuda.empty_cache()
+    assert free < 64 << 20 and held == 0
+    h.contains(kd, flags)
+    assert h.size() == n and bool((flags == 1).all())
+    c.retrieve(kd, counts)
+    assert c.size() == n and bool((counts == 1).all())
+    ob = oracle.Bloom(1 << 27, 4, 64, 64, 1, bf.seed())
+    ob.insert(keys)
+    np.testing.assert_array_equal(from_dev(bf.words(), np.uint64), ob.words())
+    assert bl.num_keys() == n // 6 and bl.num_values() == n // 6 * 6
+
+
+def test_batches_of_more_than_one_chunk(cuda):
+    """More keys than one run of the passes takes (2^28), into each kind."""
+    from warpcore_amd import _capi
+    from warpcore_amd.tables import BloomFilter, BucketListHashTable, HashSet, SingleValueHashTable
+    n = (1 << 28) + (1 << 27) + 3
+    keys = torch.empty(n, dtype=torch.int32, device="cuda")
+    assert _capi.lib().wc_gen_unique_u32(keys.data_ptr(), n, 0x9000, None) == 0
+    h = HashSet(math.ceil(n / 0.9), 32)
+    assert _sorted(lambda: h.insert(keys))
+    flags = torch.zeros(n, dtype=torch.uint8, device="cuda")
+    h.contains(keys, flags)
+    assert h.size() == n and int((flags != 1).sum()) == 0
+    del h
+    print("[chunks] set done", flush=True)
+    t = SingleValueHashTable(math.ceil(n / 0.9), 32, 32, cg_size=16)
+    st = torch.full((n,), 0x77, dtype=torch.int32, device="cuda")
+    assert _sorted(lambda: t.insert(keys, keys, status_out=st))
+    out = torch.zeros_like(keys)
+    t.retrieve(keys, out)
+    assert t.size() == n and torch.equal(out, keys) and int((st != S_NONE).sum()) == 0
+    del t, st
+    print("[chunks] table done", flush=True)
+    one, pieces = BloomFilter(1 << 30, 3, 32), BloomFilter(1 << 30, 3, 32)
+    assert _sorted(lambda: one.insert(keys))
+    for lo in range(0, n, 1 << 25):
+        pieces.insert(keys[lo:lo + (1 << 25)])
+    assert torch.equal(one.words(), pieces.words())
+    del one, pieces
+    print("[chunks] filter done", flush=True)
+    d = 1 << 24
+    owner = keys[:d].repeat(n // d + 1)[:n]
+    bl = BucketListHashTable(math.ceil(d / 0.9), 2 * n, 32, 32)
+    assert _sorted(lambda: bl.insert(owner, owner))
+    begin, end = (torch.zeros(d, dtype=torch.int64, device="cuda") for _ in range(2))
+    assert bl.retrieve(keys[:d], begin, end, out) == n
+    count = torch.full((d,), n // d, dtype=torch.int64, device="cuda")
+    count[: n % d] += 1
+    assert torch.equal(end - begin, count) and torch.equal(out, torch.repeat_interleave(keys[:d], count))
 
 
 def _streams_side_by_side():
@@ -403,6 +506,14 @@ def test_bloom_insert(cuda, oracle, kb, sb, num_bits, k, n, shape):
         np.testing.assert_array_equal(from_dev(bf.words(), dtype(sb)), ob.words())
 
 
+_WARM = [6000] * 40 + [150_000]   # pairs of the keys that overflow segments
+
+
+def _sample(n):
+    """Positions whose keys decide whether a batch is taken for skewed."""
+    return np.arange(4096) * (n // 4096)
+
+
 def _pair_batch(n, bits, distinct, shape, seed):
     """n pairs over `distinct` keys with distinct values, some keys invalid."""
     rng = np.random.default_rng(seed)
@@ -412,8 +523,9 @@ def _pair_batch(n, bits, distinct, shape, seed):
         pick = np.searchsorted(np.cumsum(w / w.sum()), rng.random(n)).clip(max=distinct - 1)
     else:
         pick = rng.integers(0, distinct, n)
-        if shape == "warm":  # a few keys of some thousand pairs, too few to be sampled
-            pick[: n // 16] = rng.integers(0, max(1, n // 16 // 3000), n // 16)
+        if shape == "warm":  # keys of some thousand pairs, none of them sampled (part_begin)
+            at = rng.permutation(np.setdiff1d(np.arange(n), _sample(n)))
+            pick[at[: sum(_WARM)]] = np.repeat(np.arange(len(_WARM)), _WARM)
     keys = uniq[pick]
     if shape == "invalid":
         keys[::9973] = 0
@@ -464,6 +576,34 @@ def test_pairs_insert(cuda, bits, n, distinct, shape):
         t.pop_status()   # key_not_found of the keys that the batch does not hold
         np.testing.assert_array_equal(got[0], want[0])
         np.testing.assert_array_equal(got[1], want[1])
+
+
+@pytest.mark.parametrize("cg,n,distinct,passes", [(4, 1_600_007, 160_000, 1), (8, 3_000_017, 300_000, 2),
+                                                  (8, 12_000_001, 1_200_000, 2)])
+def test_pairs_insert_with_overflowing_segments(cuda, cg, n, distinct, passes):
+    """Keys of 6,000 pairs, more than a region's share, and one of 150,000, more
+    than a bucket's: their records take the pair-by-pair rest (several lanes
+    append to one key at once), the others the groups."""
+    import ctypes
+    from pathlib import Path
+    from warpcore_amd.tables import BucketListHashTable
+    keys, values, uniq = _pair_batch(n, 32, distinct, "warm", seed=n)
+    assert np.unique(keys[_sample(n)], return_counts=True)[1].max() < 4   # not taken for skewed
+    t = BucketListHashTable(math.ceil(distinct / 0.9), 5 * n, 32, 32, cg_size=cg)
+    plan = (ctypes.c_uint64 * 4)()
+    ctypes.CDLL(str(Path(__file__).parent / "device_api" / "libwc_device_api.so")).wcx_group_plan(
+        ctypes.c_uint(cg), ctypes.c_uint64(n), ctypes.c_uint64(t.key_capacity()), plan)
+    cap1, cap2, buckets, two = list(plan)
+    assert two == passes - 1 and n >= t.key_capacity()
+    # an eighth of a key's pairs on each XCD, beside the mean of the others
+    assert 150_000 // 8 + n // 8 // buckets > cap1
+    if two:
+        assert 6000 > cap2
+    assert _sorted(lambda: t.insert(to_dev(keys), to_dev(values)))
+    assert int(t.pop_status()) == S_DUP
+    got, want = _values_by_key(t, uniq, 32, n), _expected_by_key(keys, values, uniq)
+    np.testing.assert_array_equal(got[0], want[0])
+    np.testing.assert_array_equal(got[1], want[1])
 
 
 @pytest.mark.parametrize("min_size,grow,max_size", [(1, 1.0, 1), (3, 1.1, 1023), (8, 2.0, 64), (1, 1.001, 1023)])
