@@ -183,9 +183,44 @@ def test_inserts_from_two_streams(cuda):
     assert t.size() == 2 * n
 
 
-def test_insert_beside_a_capture_of_another_stream(cuda):
+def test_inserts_before_under_and_after_capture(cuda):
+    """A captured insert's graph may be replayed at any time: from the capture
+    on the table's inserts are the general ones; the graph is replayed between
+    and after them."""
+    from warpcore_amd.tables import SingleValueHashTable
+    n = 2_000_000
+    keys = unique_keys(2 * n, 64, seed=22)
+    kd, vd = to_dev(keys), to_dev(_value_of(keys, 64))
+    t = SingleValueHashTable(math.ceil(2 * n / 0.9), 64, 64)
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    assert _sorted(lambda: t.insert(kd[:n], vd[:n], stream=s))
+    g = torch.cuda.CUDAGraph()
+    other = torch.zeros_like(vd[:n])
+    torch.cuda.synchronize()
+    with torch.cuda.graph(g, stream=s):
+        t.insert(kd[n:], other, stream=s)
+    out = torch.zeros_like(vd)
+    for replay in range(3):
+        other.copy_(vd[n:] + replay)
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert t.size() == 2 * n
+        t.retrieve(kd, out)
+        assert torch.equal(out[:n], vd[:n]) and torch.equal(out[n:], other)
+        assert not _sorted(lambda: t.insert(kd[:n], vd[:n], stream=s))
+        t.init(stream=s)
+        torch.cuda.synchronize()
+        assert not _sorted(lambda: t.insert(kd[:n], vd[:n], stream=s))
+
+
+@pytest.mark.parametrize("before", [False, True])
+def test_insert_beside_a_capture_of_another_stream(cuda, before):
     """A bulk insert whose workspace is allocated while another stream is
-    captured in the global mode: the insert runs, the capture stays valid."""
+    captured in the global mode: the insert runs, the capture stays valid;
+    also where the captured stream ran the region insert `before` whose end
+    the table and the workspace wait for."""
     from warpcore_amd.tables import BloomFilter, SingleValueHashTable, trim_workspace
     n = 3_000_001
     keys = unique_keys(n, 64, seed=23)
@@ -196,6 +231,8 @@ def test_insert_beside_a_capture_of_another_stream(cuda):
     g = torch.cuda.CUDAGraph()
     trim_workspace()
     torch.cuda.synchronize()
+    if before:
+        t.insert(kd, vd, stream=b)
     with torch.cuda.graph(g, stream=b, capture_error_mode="global"):
         x.add_(1)
         t.insert(kd, vd, stream=a)

@@ -1293,10 +1293,11 @@ public:
                 const bool wanted = statuses && status_out != nullptr;
                 warpcore::detail::MutationTracker::Exclusive exclusive(hash_table_.mutations_, stream);
                 index_type done = 0;
+                warpcore::detail::CompletionMark end;
                 if constexpr (warpcore::detail::part_record<warpcore::detail::PairRecord<key_type, value_type>>())
                     if (!wanted && exclusive.granted())
-                        done = insert_grouped(keys_in, values_in, num_in, stream, probing_length);
-                if (done != 0) exclusive.use();
+                        done = insert_grouped(keys_in, values_in, num_in, stream, probing_length, end);
+                if (done != 0) exclusive.use(end);
                 if (done < num_in) {
                     typename StatusHandler::base_type* out = nullptr;
                     if constexpr (statuses)
@@ -1360,7 +1361,8 @@ private:
     // where nothing else modifies the key table meanwhile; the number of
     // pairs taken (the rest is the general insert's).
     WC_H index_type insert_grouped(const key_type* keys_in, const value_type* values_in, index_type num_in,
-                                   hipStream_t stream, index_type probing_length) noexcept {
+                                   hipStream_t stream, index_type probing_length,
+                                   warpcore::detail::CompletionMark& end) noexcept {
         using key_view = typename hash_table_type::view_type;
         using core_type = detail::BucketListGroupCore<key_view, typename value_store_type::view_type>;
         using pair_type = detail::PairRecord<key_type, value_type>;
@@ -1372,7 +1374,7 @@ private:
             if (!warpcore::detail::groups_pay<pair_type>(n, keys.geometry(), stream)) break;
             const key_type* k = keys_in + done;
             const value_type* v = values_in + done;
-            if (!warpcore::detail::insert_grouped(k, v, n, core, keys, probing_length, stream,
+            if (!warpcore::detail::insert_grouped(k, v, n, core, keys, probing_length, stream, end,
                                                   [&](const index_type* count) {
                                                       insert_passes<status_handlers::ReturnNothing>(
                                                           k, v, n, stream, probing_length, nullptr, count);

@@ -734,15 +734,17 @@ private:
                 detail::owner_inserts() && n / 4 >= (index_type(1) << 20) && n / 4 >= capacity() / 8 * 3) {
                 detail::MutationTracker::Exclusive exclusive(base_table_.mutations_, stream);
                 if (!exclusive.granted()) return false;
+                detail::CompletionMark end;
                 const bool done =
                     entry_statuses<StatusHandler>(status_out)
                         ? detail::insert_partitioned_chunk<add_view_type, status_handlers::ReturnStatus, true,
                                                            typename base_type::slot_type>(
-                              buf.keys, buf.counts, n, buf.num, add_state(), probing_length, buf.status, stream)
+                              buf.keys, buf.counts, n, buf.num, add_state(), probing_length, buf.status, stream,
+                              end)
                         : detail::insert_partitioned_chunk<add_view_type, status_handlers::ReturnNothing, true,
                                                            typename base_type::slot_type>(
-                              buf.keys, buf.counts, n, buf.num, add_state(), probing_length, nullptr, stream);
-                if (done) exclusive.use();
+                              buf.keys, buf.counts, n, buf.num, add_state(), probing_length, nullptr, stream, end);
+                if (done) exclusive.use(end);
                 return done;
             }
         }

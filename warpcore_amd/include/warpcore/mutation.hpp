@@ -12,15 +12,18 @@
 //   streams: per_thread_stream), and a copy or a view of the table handed out
 //   (user kernels may modify the table through the device calls) end that;
 //   the calls that follow use the compare-and-swap paths.
-// - An exclusive call leaves an event behind its kernels. A later modifying
-//   call on another stream waits for it on the device, and handing out a copy
-//   or a view, or noting a call under capture, waits for it on the host.
+// - An exclusive call leaves an event and a mark (CompletionMark) behind its
+//   kernels. A later modifying call on another stream waits for the event on
+//   the device, and handing out a copy or a view, or noting a call under
+//   capture, waits for the mark on the host. So does a call whose wait for
+//   the event is refused: that of a stream that is captured by then.
 // - init() starts over (it fills the whole table, so a modification still
 //   running on another stream would be a race with it already), except for
 //   copies, views and graphs, which stay.
 #pragma once
 
 #include "base.hpp"
+#include "workspace.hpp"
 
 #include <mutex>
 #include <new>
@@ -36,6 +39,7 @@ class MutationTracker {
         bool shared = false;   // a copy, a view or a graph may modify the table
         hipStream_t stream = nullptr;
         hipEvent_t fence = nullptr;   // behind the last exclusive call
+        CompletionMark end;           // the same for the host
         bool fenced = false;
         hipStream_t fence_stream = nullptr;
     };
@@ -95,18 +99,20 @@ public:
         WC_H ~Exclusive() noexcept {
             if (s_ == nullptr) return;
             if (used_) {
-                if (hipEventRecord(s_->fence, stream_) == hipSuccess) {
-                    s_->fenced = true;
-                    s_->fence_stream = stream_;
-                } else {   // no event to wait for: the kernels end here
+                s_->fenced = true;
+                s_->fence_stream = stream_;
+                if (hipEventRecord(s_->fence, stream_) != hipSuccess) {   // nothing to wait for on the device
                     (void)hipGetLastError();
-                    (void)hipStreamSynchronize(stream_);
+                    wait(*s_);
                 }
             }
             s_->mu.unlock();
         }
         bool granted() const noexcept { return granted_; }
-        void use() noexcept { used_ = true; }   // exclusive kernels were enqueued
+        void use(const CompletionMark& end) noexcept {   // exclusive kernels were enqueued, which `end` is behind
+            used_ = true;
+            s_->end = end;
+        }
 
     private:
         State* s_;
@@ -117,10 +123,12 @@ public:
 private:
     WC_H void share_locked() const noexcept {
         s_->shared = true;
-        if (!s_->fenced) return;
-        const RelaxedCapture relaxed;   // also called while some stream is captured
-        (void)hipEventSynchronize(s_->fence);
-        s_->fenced = false;
+        wait(*s_);
+    }
+    // the host waits for the last exclusive call's kernels
+    WC_H static void wait(State& s) noexcept {
+        if (s.fenced) s.end.wait();
+        s.fenced = false;
     }
     // whether `stream` orders every modification
     WC_H bool note_locked(hipStream_t stream) const noexcept {
@@ -130,7 +138,11 @@ private:
             share_locked();
             return false;
         }
-        if (s_->fenced && s_->fence_stream != stream) (void)hipStreamWaitEvent(stream, s_->fence, 0);
+        if (s_->fenced && s_->end.passed()) s_->fenced = false;
+        if (s_->fenced && s_->fence_stream != stream && hipStreamWaitEvent(stream, s_->fence, 0) != hipSuccess) {
+            (void)hipGetLastError();
+            wait(*s_);
+        }
         if (per_thread_stream(stream) || (s_->any && s_->stream != stream)) s_->mixed = true;
         s_->any = true;
         s_->stream = stream;

@@ -260,7 +260,7 @@ WC_H bool groups_pay(index_t n, const probing_schemes::Geometry& geo, hipStream_
 template<class Core, class SortView, class General>
 WC_H bool insert_grouped(const typename Core::key_type* keys_in, const typename Core::pair_value_type* values_in,
                          index_t n, const Core& core, const SortView& view, index_t probing_length, hipStream_t stream,
-                         const General& general) noexcept {
+                         CompletionMark& end, const General& general) noexcept {
     using K = typename Core::key_type;
     using V = typename Core::pair_value_type;
     using Rec = PairRecord<K, V>;
@@ -269,7 +269,7 @@ WC_H bool insert_grouped(const typename Core::key_type* keys_in, const typename 
     const PartPlan p = make_part_plan<Sort, Rec, false>(n, core.geometry(), group_windows<Core, Rec>(n, core.geometry()),
                                                         kGroupSigmas);
     if (p.regions == 0) return false;
-    WorkspaceLease ws(p.bytes + sizeof(index_t), stream);   // and the general insert's count
+    WorkspaceLease ws(p.bytes + sizeof(index_t), stream, &end);   // and the general insert's count
     if (!ws) return false;
     auto* at = static_cast<unsigned char*>(ws.get());
     auto* A = reinterpret_cast<Rec*>(at + p.a);

@@ -890,18 +890,19 @@ WC_H bool partition_pays(index_t n, const probing_schemes::Geometry& geo) noexce
     return n >= least && n >= geo.capacity / 8 * eighths && n <= 2 * geo.capacity && geo.windows < (index_t(1) << 31);
 }
 
-// Runs the passes over one chunk; false (nothing launched) without a
-// workspace for it. With num_dev the chunk holds min(n, *num_dev) keys (a
+// Runs the passes over one chunk, `end` behind them; false (nothing launched)
+// without a workspace for it. With num_dev the chunk holds min(n, *num_dev) keys (a
 // count made on the device), none of them frequent, so none are sampled.
 template<class Core, class StatusHandler, bool HasValues, class Rec>
 WC_H bool insert_partitioned_chunk(const typename Core::key_type* keys_in, const typename Core::value_type* values_in,
                                    index_t n, const index_t* num_dev, const Core& core, index_t probing_length,
-                                   typename StatusHandler::base_type* status_out, hipStream_t stream) noexcept {
+                                   typename StatusHandler::base_type* status_out, hipStream_t stream,
+                                   CompletionMark& end) noexcept {
     using V = typename Core::value_type;
     constexpr bool Idx = !std::is_same<StatusHandler, status_handlers::ReturnNothing>::value;
     const PartPlan p = make_part_plan<Core, Rec, Idx>(n, core.geometry());
     if (p.regions == 0) return false;
-    WorkspaceLease ws(p.bytes, stream);
+    WorkspaceLease ws(p.bytes, stream, &end);
     if (!ws) return false;
     auto* at = static_cast<unsigned char*>(ws.get());
     auto* A = reinterpret_cast<Rec*>(at + p.a);
@@ -954,7 +955,8 @@ WC_H bool insert_partitioned_chunk(const typename Core::key_type* keys_in, const
 template<class Core, class StatusHandler, bool HasValues, class Rec>
 WC_H index_t insert_partitioned(const typename Core::key_type* keys_in, const typename Core::value_type* values_in,
                                 index_t n, const Core& core, index_t probing_length,
-                                typename StatusHandler::base_type* status_out, hipStream_t stream) noexcept {
+                                typename StatusHandler::base_type* status_out, hipStream_t stream,
+                                CompletionMark& end) noexcept {
     index_t done = 0;
     while (done < n) {
         const index_t m = n - done < kPartChunk ? n - done : kPartChunk;
@@ -963,7 +965,7 @@ WC_H index_t insert_partitioned(const typename Core::key_type* keys_in, const ty
         if constexpr (!std::is_same<StatusHandler, status_handlers::ReturnNothing>::value)
             if (status_out != nullptr) st = status_out + done;
         if (!insert_partitioned_chunk<Core, StatusHandler, HasValues, Rec>(
-                keys_in + done, HasValues ? values_in + done : nullptr, m, nullptr, core, probing_length, st, stream))
+                keys_in + done, HasValues ? values_in + done : nullptr, m, nullptr, core, probing_length, st, stream, end))
             break;
         done += m;
     }
@@ -987,10 +989,11 @@ WC_H bool insert_partitioned_first(const MutationTracker& mutations, const typen
     }
     MutationTracker::Exclusive exclusive(mutations, stream);
     if (!exclusive.granted()) return false;
+    CompletionMark end;
     const index_t done = insert_partitioned<Core, StatusHandler, HasValues, Rec>(
-        keys_in, values_in, num_in, core, probing_length, status_out, stream);
+        keys_in, values_in, num_in, core, probing_length, status_out, stream, end);
     if (done == 0) return false;
-    exclusive.use();
+    exclusive.use(end);
     keys_in += done;
     if constexpr (HasValues) values_in += done;
     num_in -= done;

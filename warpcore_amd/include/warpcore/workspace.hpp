@@ -1,9 +1,9 @@
 // Scratch memory of bulk calls, shared by all tables of the process.
 //
 // A bulk call leases one buffer for the kernels it launches. The lease ends
-// with the call, and an event is recorded behind the call's kernels. A buffer
-// is handed out again to a call on the same stream, or once that event has
-// passed: no stream ever waits for another one's work here, calls on several
+// with the call, whose last kernel writes a mark that the host can read. A buffer
+// is handed out again to a call on the same stream, or once that mark is
+// there: no stream ever waits for another one's work here, calls on several
 // streams or host threads get buffers of their own. Bounded: at most
 // kWorkspaceLimit bytes per device; a lease that would exceed it, or that
 // finds no device memory, is empty and the caller runs its kernels that need
@@ -22,10 +22,36 @@
 
 #include <mutex>
 #include <new>
+#include <thread>
 
 namespace warpcore {
+
+namespace kernels {
+
+// Behind a call's other kernels: they are over. (Their writes reached memory
+// when they ended; the store alone is for the host.)
+__global__ inline void complete(std::uint64_t* word, std::uint64_t seq) {
+    __hip_atomic_store(word, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+}  // namespace kernels
+
 namespace detail {
 
+// The end of some kernels, as the host reads it without a call to the runtime:
+// a query of an event, or a wait for one, ends a capture of the stream on which
+// the event was recorded, however long before.
+struct CompletionMark {
+    std::uint64_t* word = nullptr;   // in pinned host memory; it only grows
+    std::uint64_t seq = 0;
+
+    WC_H bool passed() const noexcept { return word == nullptr || __atomic_load_n(word, __ATOMIC_ACQUIRE) >= seq; }
+    WC_H void wait() const noexcept {
+        while (!passed()) std::this_thread::yield();
+    }
+};
+
+constexpr unsigned kMarkWords = 512;   // of 8 bytes; as many buffers at once at most
 constexpr std::size_t kWorkspaceLimit = std::size_t(16) << 30;
 constexpr std::size_t kWorkspaceUnit = std::size_t(1) << 20;   // leases are rounded up to this
 
@@ -42,7 +68,7 @@ public:
         void* p = nullptr;
         std::size_t bytes = 0;
         int device = 0;
-        hipEvent_t done = nullptr;   // behind the last user's kernels
+        CompletionMark done;         // behind the last user's kernels
         hipStream_t stream = nullptr;   // the last user's
         bool leased = false;
         Buffer* next = nullptr;
@@ -70,14 +96,9 @@ public:
         Buffer* best = nullptr;
         for (Buffer* b = first_; b != nullptr; b = b->next)
             if (!b->leased && b->device == device && b->bytes >= bytes &&
-                (best == nullptr || b->bytes < best->bytes) && (ordered(b, stream) || passed(b)))
+                (best == nullptr || b->bytes < best->bytes) && (ordered(b, stream) || b->done.passed()))
                 best = b;
         if (best != nullptr) {
-            // (nothing to wait for unless the handle was given to a new stream)
-            if (hipStreamWaitEvent(stream, best->done, 0) != hipSuccess) {
-                (void)hipGetLastError();
-                return nullptr;
-            }
             best->leased = true;
             return best;
         }
@@ -89,15 +110,12 @@ public:
         if (b == nullptr) return nullptr;
         b->bytes = bytes;
         b->device = device;
-        if (hipEventCreateWithFlags(&b->done, hipEventDisableTiming) != hipSuccess) {
-            (void)hipGetLastError();
-            delete b;
-            return nullptr;
-        }
+        b->done.word = take_word();
+        if (b->done.word != nullptr) b->done.seq = *b->done.word;
         if (available_gpu_memory() / 2 < bytes) free_idle(device);
-        if (available_gpu_memory() / 2 < bytes || hipMalloc(&b->p, bytes) != hipSuccess) {
+        if (b->done.word == nullptr || available_gpu_memory() / 2 < bytes || hipMalloc(&b->p, bytes) != hipSuccess) {
             (void)hipGetLastError();
-            (void)hipEventDestroy(b->done);
+            give_word(b->done.word);
             delete b;
             return nullptr;
         }
@@ -106,16 +124,23 @@ public:
         first_ = b;
         return b;
     }
-    WC_H void release(Buffer* b, hipStream_t stream) noexcept {
+    // the end of the kernels enqueued on `stream` so far
+    WC_H CompletionMark release(Buffer* b, hipStream_t stream) noexcept {
         std::lock_guard<std::mutex> lock(mu_);
         const RelaxedCapture relaxed;
-        if (hipEventRecord(b->done, stream) != hipSuccess) {
+        ++b->done.seq;
+        void* args[] = {&b->done.word, &b->done.seq};
+        if (hipLaunchKernel(reinterpret_cast<const void*>(kernels::complete), dim3(1), dim3(1), args, 0, stream) !=
+            hipSuccess) {
             (void)hipGetLastError();
-            (void)hipStreamSynchronize(stream);   // no event to wait for: the kernels end here
+            (void)hipStreamSynchronize(stream);   // nobody to write the mark: the kernels end here
+            __atomic_store_n(b->done.word, b->done.seq, __ATOMIC_RELEASE);
         }
         b->stream = stream;
         b->leased = false;
+        const CompletionMark done = b->done;
         if (users_ == 0) free_idle(-1);
+        return done;
     }
     // frees the buffers no call holds, after waiting for the kernels that
     // still use them; the bytes freed, on all devices
@@ -133,13 +158,31 @@ public:
     }
 
 private:
+    // (destroying a stream waits for its work on this runtime, so a new stream
+    // that is given an old one's handle is ordered behind it too)
     WC_H static bool ordered(const Buffer* b, hipStream_t stream) noexcept {
         return b->stream == stream && !per_thread_stream(stream);
     }
-    WC_H static bool passed(const Buffer* b) noexcept {
-        const hipError_t e = hipEventQuery(b->done);
-        if (e != hipSuccess && hipPeekAtLastError() == e) (void)hipGetLastError();
-        return e == hipSuccess;
+    // a word of the marks' memory, allocated with the first; null when all are in use
+    WC_H std::uint64_t* take_word() noexcept {
+        if (words_ == nullptr) {
+            if (hipHostMalloc(reinterpret_cast<void**>(&words_), kMarkWords * sizeof(std::uint64_t),
+                              hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess) {
+                (void)hipGetLastError();
+                words_ = nullptr;
+                return nullptr;
+            }
+            for (unsigned w = 0; w < kMarkWords; ++w) words_[w] = 0;
+        }
+        for (unsigned w = 0; w < kMarkWords; ++w)
+            if (!taken_[w]) {
+                taken_[w] = true;
+                return words_ + w;
+            }
+        return nullptr;
+    }
+    WC_H void give_word(std::uint64_t* word) noexcept {
+        if (word != nullptr) taken_[word - words_] = false;
     }
     // bytes of one device's buffers, or (-1) of all
     WC_H std::size_t held_on(int device) const noexcept {
@@ -153,19 +196,21 @@ private:
     WC_H void free_idle(int device) noexcept {
         for (Buffer** at = &first_; *at != nullptr;) {
             Buffer* b = *at;
-            if (b->leased || (device >= 0 && (b->device != device || !passed(b)))) {
+            if (b->leased || (device >= 0 && (b->device != device || !b->done.passed()))) {
                 at = &b->next;
                 continue;
             }
             *at = b->next;
-            (void)hipEventSynchronize(b->done);
+            b->done.wait();
             (void)hipFree(b->p);
-            (void)hipEventDestroy(b->done);
+            give_word(b->done.word);
             delete b;
         }
     }
 
     std::mutex mu_;
+    std::uint64_t* words_ = nullptr;   // marks; kept: trackers read theirs after the buffer is gone
+    bool taken_[kMarkWords] = {};
     Buffer* first_ = nullptr;   // linked in the buffers themselves: a lease allocates nothing that may throw
     std::size_t users_ = 0;
 };
@@ -184,15 +229,18 @@ WC_H hipError_t device_malloc(T** p, std::size_t bytes) noexcept {
     return hipMalloc(reinterpret_cast<void**>(p), bytes);
 }
 
-// One bulk call's lease; false when the pool has no buffer for it.
+// One bulk call's lease; false when the pool has no buffer for it. `end` (may
+// be null) becomes the mark behind the call's kernels.
 class WorkspaceLease {
 public:
-    WC_H WorkspaceLease(std::size_t bytes, hipStream_t stream) noexcept
-        : buffer_(WorkspacePool::instance().acquire(bytes, stream)), stream_(stream) {}
+    WC_H WorkspaceLease(std::size_t bytes, hipStream_t stream, CompletionMark* end = nullptr) noexcept
+        : buffer_(WorkspacePool::instance().acquire(bytes, stream)), stream_(stream), end_(end) {}
     WorkspaceLease(const WorkspaceLease&) = delete;
     WorkspaceLease& operator=(const WorkspaceLease&) = delete;
     WC_H ~WorkspaceLease() noexcept {
-        if (buffer_ != nullptr) WorkspacePool::instance().release(buffer_, stream_);
+        if (buffer_ == nullptr) return;
+        const CompletionMark done = WorkspacePool::instance().release(buffer_, stream_);
+        if (end_ != nullptr) *end_ = done;
     }
     explicit operator bool() const noexcept { return buffer_ != nullptr; }
     void* get() const noexcept { return buffer_ != nullptr ? buffer_->p : nullptr; }
@@ -200,6 +248,7 @@ public:
 private:
     WorkspacePool::Buffer* buffer_;
     hipStream_t stream_;
+    CompletionMark* end_;
 };
 
 }  // namespace detail
