@@ -36,3 +36,9 @@ def test_grids_are_multiples_of_the_xcds(resident):
         units = 100
         taken = sorted((v, b % 8) for b in range(grid) for v in range(b // 8, units, grid // 8))
         assert taken == [(v, x) for v in range(units) for x in range(8)]
+
+
+def test_copies_of_a_table_keep_its_mutation_state():
+    """A copy is copied after its table is gone: the state they share is
+    deleted once, with the last of them."""
+    assert _lib("host_memory").wch_tracker_lifetime() == 1

@@ -193,7 +193,6 @@ public:
         if (!is_copy_) {
             if (keys_ != nullptr) (void)hipFree(keys_);
             if (status_ != nullptr) (void)hipFree(status_);
-            mutations_.destroy();
             detail::WorkspacePool::instance().remove_user();
         }
 #endif

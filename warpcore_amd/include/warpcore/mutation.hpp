@@ -25,6 +25,7 @@
 #include "base.hpp"
 #include "workspace.hpp"
 
+#include <atomic>
 #include <mutex>
 #include <new>
 
@@ -33,6 +34,7 @@ namespace detail {
 
 class MutationTracker {
     struct State {
+        std::atomic<unsigned> holders{1};   // host objects
         std::mutex mu;
         bool any = false;      // `stream` is the one that ordered every modification so far
         bool mixed = false;    // more than one stream since the last init()
@@ -46,16 +48,20 @@ class MutationTracker {
 
 public:
     WC_H MutationTracker() noexcept : s_(new (std::nothrow) State) {}
-    // a shallow copy of the table: it shares the state, which its owner destroys
-    WC_HD MutationTracker(const MutationTracker& o) noexcept : s_(o.s_) { share(); }
-    WC_H MutationTracker(MutationTracker&& o) noexcept : s_(o.s_) {}
+    // a shallow copy of the table shares the state, which lives as long as the
+    // last of them on the host (a copy may be copied after its table is gone)
+    WC_HD MutationTracker(const MutationTracker& o) noexcept : s_(o.s_) {
+        hold();
+        share();
+    }
+    WC_H MutationTracker(MutationTracker&& o) noexcept : s_(o.s_) { hold(); }
     MutationTracker& operator=(const MutationTracker&) = delete;
-
-    WC_H void destroy() noexcept {   // by the table that owns the state
-        if (s_ == nullptr) return;
+    WC_HD ~MutationTracker() noexcept {
+#if !defined(__HIP_DEVICE_COMPILE__)
+        if (s_ == nullptr || s_->holders.fetch_sub(1, std::memory_order_acq_rel) != 1) return;
         if (s_->fence != nullptr) (void)hipEventDestroy(s_->fence);
         delete s_;
-        s_ = nullptr;
+#endif
     }
 
     WC_HD void share() const noexcept {
@@ -121,6 +127,11 @@ public:
     };
 
 private:
+    WC_HD void hold() const noexcept {
+#if !defined(__HIP_DEVICE_COMPILE__)
+        if (s_ != nullptr) s_->holders.fetch_add(1, std::memory_order_relaxed);
+#endif
+    }
     WC_H void share_locked() const noexcept {
         s_->shared = true;
         wait(*s_);

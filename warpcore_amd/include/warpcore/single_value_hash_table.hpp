@@ -492,10 +492,7 @@ public:
 #if !defined(__HIP_DEVICE_COMPILE__)
         if (!is_copy_ && status_ != nullptr) (void)hipFree(status_);
         if (!is_copy_ && filter_ != nullptr) (void)hipFree(filter_);
-        if (!is_copy_) {
-            mutations_.destroy();
-            detail::WorkspacePool::instance().remove_user();
-        }
+        if (!is_copy_) detail::WorkspacePool::instance().remove_user();
 #endif
     }
 
