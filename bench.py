@@ -58,15 +58,16 @@ def algorithmic_bytes(op: str, kb: int, vb: int) -> int:
 
 
 def region_bytes(rec: int, table_bytes: int, n: int, passes: int) -> int:
-    """Bytes per key of an insert sorted by table region: records of `rec`
-    bytes read, written and read once more by each sorting pass, the table
-    streamed in and out."""
+    """Bytes per key that an insert sorted by table region streams, as a model:
+    records of `rec` bytes read, written and read once more by each sorting
+    pass, the table in and out. The random lines of keys whose first window is
+    full are not in it (measured traffic: read_traffic)."""
     return round(rec * (1 + 2 * passes) + 2 * table_bytes / n)
 
 
 # Revision of the probing kernels' code; a traffic figure measured on
 # another revision is not used.
-KERNEL_REVISION = "owner-4"
+KERNEL_REVISION = "regions-1"
 
 
 def read_traffic(family: str, log2n: int = 28, table: str = "u64"):
@@ -99,12 +100,16 @@ def kernel_family(lib, op: str) -> str:
     return "retrieve_lockstep" if k & 2 else "retrieve_batched"
 
 
-def bulk_family(lib, op: str, n: int) -> str:
-    """The same for a call of n keys that fill most of an empty table: such
-    inserts of at least 2^20 keys run the region passes (part_scatter,
-    part_refine, part_build, part_tail), not the lane-owner kernel alone."""
+def bulk_family(lib, op: str, n: int, capacity: int, slot_bytes: int = 16) -> str:
+    """The same for a call of n keys on a table that one stream modifies:
+    inserts of at least 2^20 keys and a quarter (8-byte slots) or three eighths
+    of the slots, at most twice them, run the region passes (part_scatter,
+    part_refine, part_build, part_tail), not the lane-owner kernel alone
+    (partition_pays in partition.hpp)."""
     family = kernel_family(lib, op)
-    return "insert_partitioned" if family == "insert_owner" and n >= 1 << 20 else family
+    eighths = 3 if slot_bytes > 8 else 2
+    sorted_ = n >= 1 << 20 and capacity // 8 * eighths <= n <= 2 * capacity
+    return "insert_partitioned" if family == "insert_owner" and sorted_ else family
 
 
 def probes_lib():
@@ -786,7 +791,7 @@ def main():
 
     n = r64["n"]
     per_op = {"insert": algorithmic_bytes("insert", 64, 64), "retrieve": algorithmic_bytes("retrieve", 64, 64)}
-    fam = {op: bulk_family(g.lib, op, n) for op in ("insert", "retrieve")}
+    fam = {op: bulk_family(g.lib, op, n, r64["capacity"]) for op in ("insert", "retrieve")}
     if fam["insert"] == "insert_partitioned":
         per_op["insert"] = region_bytes(16, r64["table_bytes"], n, 2)
     kt = {"insert": r64["insert_ms"], "retrieve": r64["retrieve_ms"]}
@@ -818,7 +823,7 @@ def main():
     if "u32u32_cg16" in extras:   # the same for the u32 table (2.4 GB of 8-byte slots)
         lr32 = run_line_roofline(g, r32["table_bytes"])
         for op in ("retrieve", "insert"):
-            tr = read_traffic(fam[op], args.log2_keys, "u32")
+            tr = read_traffic(bulk_family(g.lib, op, r32["n"], r32["capacity"], 8), args.log2_keys, "u32")
             if tr:
                 lines_per_op = tr / LINE / r32["n"]
                 lr32[f"{op}_lines_per_op"] = round(lines_per_op, 3)

@@ -37,3 +37,21 @@ def test_probe_library_binding():
         build_probes()
     lib = bench.probes_lib()
     assert hasattr(lib, "wc_util_gather_lines")
+
+
+def test_bulk_family_follows_the_fill_rule():
+    lib = _Lib(220)
+    assert bench.bulk_family(lib, "insert", 1 << 28, 298_876_376) == "insert_partitioned"
+    assert bench.bulk_family(lib, "insert", 3 << 20, 8 << 20) == "insert_partitioned"
+    assert bench.bulk_family(lib, "insert", (3 << 20) - 1, 8 << 20) == "insert_owner"
+    assert bench.bulk_family(lib, "insert", 2 << 20, 8 << 20, slot_bytes=8) == "insert_partitioned"
+    assert bench.bulk_family(lib, "insert", (1 << 20) - 1, 1 << 20) == "insert_owner"
+    assert bench.bulk_family(lib, "insert", (2 << 20) + 1, 1 << 20) == "insert_owner"
+    assert bench.bulk_family(lib, "retrieve", 1 << 28, 298_876_376) == "retrieve_owner"
+    assert bench.bulk_family(_Lib(28), "insert", 1 << 28, 298_876_376) == "insert_refill"
+
+
+def test_region_traffic_is_measured_for_both_headline_tables():
+    for table in ("u64", "u32"):
+        for family in ("insert_partitioned", "retrieve_owner"):
+            assert bench.read_traffic(family, table=table) > 1e10

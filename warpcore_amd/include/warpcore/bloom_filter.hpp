@@ -35,7 +35,8 @@ namespace warpcore {
 namespace detail {
 
 // Partitioned insert: keys per thread of a tile, most regions (whose LDS
-// bounds a region by kRegionBytes, the filter by 128 MB).
+// bounds a region by kRegionBytes, the filter by 128 MB; more regions, which
+// the tile's LDS would hold, were not measured).
 constexpr unsigned kBloomItems = 8;
 constexpr unsigned kBloomRegions = 2048;
 
